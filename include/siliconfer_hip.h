@@ -158,6 +158,16 @@ int sf_q4_gemm(const void *blob, const void *x, int x_dtype, void *y, int y_dtyp
                const void *bias, int bias_dtype, int M, int N, int K, int group_size,
                int has_zeros, void *workspace, size_t workspace_bytes, void *stream);
 
+/* Y = X . dequant(W)^T for any M, on whichever kernel is the fastest for the
+ * shape: sf_q4_gemv's for few rows (bias may then be y_f32 itself), the tile
+ * kernels above that. Arguments and results as sf_q4_gemm. workspace:
+ * sf_q4_matmul_workspace_bytes(...) bytes, 16-byte aligned (may be 0 -> NULL
+ * ok): K-split partials and, for fp32 X, its bf16 high and low halves. */
+size_t sf_q4_matmul_workspace_bytes(int M, int N, int K, int group_size, int x_dtype);
+int sf_q4_matmul(const void *blob, const void *x, int x_dtype, void *y, int y_dtype, float *y_f32,
+                 const void *bias, int bias_dtype, int M, int N, int K, int group_size,
+                 int has_zeros, void *workspace, size_t workspace_bytes, void *stream);
+
 /* The prefill GEMM with its K-split partials left for the next op (no
  * counterpart in the reference, whose q4_gemm returns Y; here the decoder's
  * prompt path folds the residual delta into the RMSNorm that follows).

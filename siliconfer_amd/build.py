@@ -32,7 +32,9 @@ HIPCC_FLAGS = [
 # Per-file flags. The attention kernels' MFMA results stay in ordinary VGPRs
 # (without this the compiler keeps them in AGPRs and moves them back and forth
 # around the softmax and the accumulator rescaling; measured 1.5% faster).
-FILE_FLAGS = {"kv_attn.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
+_VGPR_FORM = ["-mllvm", "-amdgpu-mfma-vgpr-form"]
+FILE_FLAGS = {f: _VGPR_FORM for f in ("kv_attn.hip", "q4_gemm_rows_f16.hip", "q4_gemm_rows_bf16.hip",
+                                      "q4_gemm_rows_f32.hip")}
 
 
 def _hipcc() -> str:

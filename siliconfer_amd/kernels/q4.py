@@ -2,9 +2,9 @@
 
 `Q4Weight` owns the device blob that `sf_q4_repack` builds from the reference's
 canonical packed tensors (siliconfer/kernels/neon/__init__.py:42-81). Its
-`matmul` routes rows <= 8 to the decode GEMV where its MFMA plan takes the
-shape (sf_q4_gemv_supported) and everything else to the prefill GEMM — the
-roles of q4_gemv_* and q4_gemm_* in the reference
+`matmul` runs few rows on the decode GEMV and more on the prefill GEMM
+(sf_q4_matmul picks the kernel) — the roles of q4_gemv_* and q4_gemm_* in the
+reference
 (siliconfer/kernels/neon/bindings.cpp:45-150). Every K and group size the
 reference takes (K % group_size == 0) computes.
 """
@@ -112,16 +112,10 @@ class Q4Weight:
         st = _lib.stream(x)
         ydt = _lib.dt(out) if out is not None else _lib.SF_F32
         bdt = _lib.dt(bias) if bias is not None else 0
-        if M <= GEMV_MAX_ROWS and lib.sf_q4_gemv_supported(M, N, K, g, _lib.dt(x)):
-            rc = lib.sf_q4_gemv(self.blob.data_ptr(), x.data_ptr(), _lib.dt(x), _lib.ptr(out), ydt,
-                                _lib.ptr(out_f32), _lib.ptr(bias), bdt, M, N, K, g,
-                                int(self.has_zeros), st)
-            _lib.check(rc, "sf_q4_gemv")
-        else:
-            ws_bytes = lib.sf_q4_gemm_workspace_bytes(M, N, K, g)
-            ws = torch.empty(ws_bytes, dtype=torch.uint8, device=x.device) if ws_bytes else None
-            rc = lib.sf_q4_gemm(self.blob.data_ptr(), x.data_ptr(), _lib.dt(x), _lib.ptr(out), ydt,
-                                _lib.ptr(out_f32), _lib.ptr(bias), bdt, M, N, K, g,
-                                int(self.has_zeros), _lib.ptr(ws), ws_bytes, st)
-            _lib.check(rc, "sf_q4_gemm")
+        ws_bytes = lib.sf_q4_matmul_workspace_bytes(M, N, K, g, _lib.dt(x))
+        ws = torch.empty(ws_bytes, dtype=torch.uint8, device=x.device) if ws_bytes else None
+        rc = lib.sf_q4_matmul(self.blob.data_ptr(), x.data_ptr(), _lib.dt(x), _lib.ptr(out), ydt,
+                              _lib.ptr(out_f32), _lib.ptr(bias), bdt, M, N, K, g,
+                              int(self.has_zeros), _lib.ptr(ws), ws_bytes, st)
+        _lib.check(rc, "sf_q4_matmul")
         return out if out is not None else out_f32

@@ -179,8 +179,9 @@ class LlamaModel:
         ws = 0
         for w in (L0.qkv, L0.o, L0.gate_up, L0.down):
             for M in range(1, max(max_prefill, self.VERIFY_ROWS) + 1):
-                ws = max(ws, self.lib.sf_q4_gemm_workspace_bytes(M, w.out_features, w.in_features,
-                                                                 w.group_size))
+                ws = max(ws, self._ws_need(w, M),
+                         self.lib.sf_q4_gemm_workspace_bytes(M, w.out_features, w.in_features,
+                                                             w.group_size))
         self._gemm_ws = torch.empty(ws, dtype=torch.uint8, device=dev) if ws else None
 
     def sibling(self) -> "LlamaModel":
@@ -290,25 +291,22 @@ class LlamaModel:
 
     def _gemm(self, w: Q4Weight, X: torch.Tensor, Y32: torch.Tensor, bias: torch.Tensor | None):
         M = X.shape[0]
-        if self._gemv_ok(M, w):
-            # up to 8 rows (a short chunk, a speculative verify): the batch GEMV
-            # streams the weights once for all rows
-            self._chk(self.lib.sf_q4_gemv(w.blob.data_ptr(), X.data_ptr(), _DT[X.dtype], None,
-                                          _lib.SF_F32, Y32.data_ptr(),
-                                          None if bias is None else bias.data_ptr(), _lib.SF_F32, M,
-                                          w.out_features, w.in_features, w.group_size,
-                                          int(w.has_zeros), self._st()), "sf_q4_gemv")
-            return
-        need = self.lib.sf_q4_gemm_workspace_bytes(M, w.out_features, w.in_features, w.group_size)
+        need = self._ws_need(w, M)
         if need and (self._gemm_ws is None or self._gemm_ws.numel() < need):
             raise SFError(f"GEMM workspace: {need} bytes for {M} rows exceeds the preallocated "
                           f"{0 if self._gemm_ws is None else self._gemm_ws.numel()} (max_prefill)")
         ws = self._gemm_ws if need else None
-        self._chk(self.lib.sf_q4_gemm(w.blob.data_ptr(), X.data_ptr(), _DT[X.dtype], None, _lib.SF_F32,
-                                      Y32.data_ptr(), None if bias is None else bias.data_ptr(),
-                                      _lib.SF_F32, M, w.out_features, w.in_features, w.group_size,
-                                      int(w.has_zeros), None if ws is None else ws.data_ptr(),
-                                      0 if ws is None else ws.numel(), self._st()), "sf_q4_gemm")
+        # up to 8 rows (a short chunk, a speculative verify) this is the batch
+        # GEMV, which streams the weights once for all rows
+        self._chk(self.lib.sf_q4_matmul(w.blob.data_ptr(), X.data_ptr(), _DT[X.dtype], None, _lib.SF_F32,
+                                        Y32.data_ptr(), None if bias is None else bias.data_ptr(),
+                                        _lib.SF_F32, M, w.out_features, w.in_features, w.group_size,
+                                        int(w.has_zeros), None if ws is None else ws.data_ptr(),
+                                        0 if ws is None else ws.numel(), self._st()), "sf_q4_matmul")
+
+    def _ws_need(self, w: Q4Weight, M: int) -> int:
+        return int(self.lib.sf_q4_matmul_workspace_bytes(M, w.out_features, w.in_features, w.group_size,
+                                                         _DT[self.act_dtype]))
 
     def _gemm_parts(self, w: Q4Weight, X: torch.Tensor) -> int:
         """Where the GEMM splits K for these rows, run it leaving its partials
@@ -318,7 +316,10 @@ class LlamaModel:
         if M <= GEMM_GEMV_ROWS and self._gemv_ok(min(M, 8), w):
             return 0  # sf_q4_gemm runs these rows as 8-row batch GEMVs: no partials
         S = int(self.lib.sf_q4_gemm_splits(M, w.out_features, w.in_features, w.group_size))
-        if S <= 1:
+        # two splits: the unsplit tiles of _gemm are faster (512 x 896 x 896 fp16
+        # 7.4 us against 10.1); fp32 activations: _gemm splits them into halves
+        # once, the partials kernel in every tile
+        if S <= 2 or self.act_dtype == torch.float32:
             return 0
         need = self.lib.sf_q4_gemm_workspace_bytes(M, w.out_features, w.in_features, w.group_size)
         if self._gemm_ws is None or self._gemm_ws.numel() < need:
