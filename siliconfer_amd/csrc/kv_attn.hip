@@ -972,6 +972,292 @@ k_attn_prefill_mfma(const void *__restrict__ q, const int8_t *__restrict__ kc,
   }
 }
 
+// ---------------------------------------------------------------------------
+// causal prefill attention, 32 query rows per workgroup
+// ---------------------------------------------------------------------------
+// k_attn_prefill_mfma's scheme (waves take the 32-key tiles round robin, each
+// with its own online softmax; exact codes, q and P as fp16 high + low parts,
+// masked keys weigh exactly 0) on v_mfma_f32_32x32x16_f16: the conversion of a
+// tile's codes, about half of that kernel's VALU work, serves 32 rows instead
+// of 16. S^T = K Q^T leaves each lane 16 keys of one row, keys 8 (e / 4) + 4 h +
+// e % 4 (h = lane / 32), which are the B operands of O^T = V^T P^T as they
+// stand once V's keys are taken in the same order (slice s, half h: keys
+// 16 s + {4 h .. 4 h + 3, 8 + 4 h .. 8 + 4 h + 3}). K's dims are taken 16 per
+// half, so a lane's codes are whole 16-byte loads. A tile's registers are
+// loaded again as soon as their bytes are in LDS or operands (the next tile's
+// loads fly during this one's softmax and products). O is rescaled only when
+// some row's maximum moved (the factor is exactly 1 otherwise), and tiles wholly
+// inside every row's limit skip the masks. Bound by VALU issue and the latency of
+// a wave's chain (products, softmax, products), three waves a SIMD beside each
+// other. Measured against k_attn_prefill_mfma (us, fp32 q): 1500 rows behind 300
+// at 32 / 8 heads of 128 142 -> 74.5, 512 rows 26.8 -> 16.3; 1500 rows at 14 / 2
+// heads of 64 29.8 -> 23.7. Relative error against 64 bits 4.8e-6 -> 0.4e-6 (the
+// scaled weights). Tried: 128 rows a workgroup with the conversions shared
+// through LDS and a barrier a tile (177 us: one wave a SIMD, nothing to hide its
+// chain); V through registers (110: spills at head_dim 128).
+template <int QDT, int SDT, int D>
+__global__ void __launch_bounds__(256, 2)
+k_attn_prefill_rows(const void *__restrict__ q, const int8_t *__restrict__ kc,
+                    const void *__restrict__ ks, const int8_t *__restrict__ vc,
+                    const void *__restrict__ vs, void *__restrict__ out, int odt, int H, int KVH,
+                    int T_q, int T0, const int *__restrict__ T0_dev, int T_cap, float qscale) {
+  static_assert(D == 64 || D == 128, "head_dim 64 or 128");
+  constexpr int NW = 4;
+  constexpr int NF = D / 16;       // operand fragments of K (16 dims each) and of V (32 dims x 16 keys)
+  constexpr int NDB = D / 32;      // 32-dim blocks
+  constexpr int VC = D / 32;       // 1 KB loads of a V tile
+  constexpr bool QSPLIT = QDT != SF_F16;
+  typedef float float16_t __attribute__((ext_vector_type(16)));
+  // Each wave's V tiles, two in turn in arrays of their own (so that reading one
+  // does not wait for the loads into the other), row r's 16-byte piece p in
+  // place p ^ (r % (D / 16)): the transposing reads take one piece of eight
+  // rows. And its scales: K scale * qscale, V scale.
+  __shared__ __attribute__((aligned(16))) uint8_t v0[NW][32 * D], v1[NW][32 * D];
+  __shared__ __attribute__((aligned(16))) float scl[NW][2][32];
+
+  const int kvh = (int)(blockIdx.x % (unsigned)KVH);
+  const int G = H / KVH;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int l32 = lane & 31, h = lane >> 5;
+  const int ncol = T_q * G;
+  const int nblk = (ncol + 31) >> 5;
+  const int c0 = (nblk - 1 - (int)(blockIdx.x / (unsigned)KVH)) * 32;  // longest rows first
+  const int start = T0_dev ? *T0_dev : T0;
+  auto limit = [&](int c) { return max(0, min(start + c / G + 1, T_cap)); };  // keys column c sees
+  const int c = min(c0 + l32, ncol - 1);  // columns past the rows repeat the last one (not stored)
+  const int lim = limit(c);
+  const int lo = limit(c0), t1 = limit(min(c0 + 31, ncol - 1));  // the first and the last row's
+  const size_t base = (size_t)kvh * T_cap;
+  const size_t qrow = (size_t)(c / G) * H + (size_t)kvh * G + c % G;
+
+  // q: fragment f holds dims 32 (f / 2) + 16 h + 8 (f % 2) .. + 7 of the lane's
+  // row; in registers at head_dim 64, in LDS (made once, wave w fragments
+  // f % 4 == w) at 128, where they would not fit beside the output
+  constexpr bool QLDS = D == 128;
+  __shared__ __attribute__((aligned(16))) half8_t qs[QLDS ? NF * (QSPLIT ? 2 : 1) : 1][QLDS ? 64 : 1];
+  half8_t qr[QLDS ? 1 : NF][2];
+  auto make_q = [&](int f, half8_t &hi, half8_t &lo) {
+    float v[8];
+    sf_load8_as_f32<QDT>(q, qrow * D + 32 * (f >> 1) + 16 * h + 8 * (f & 1), v);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      hi[i] = (f16)v[i];
+      lo[i] = (f16)(v[i] - (float)hi[i]);
+    }
+  };
+  if constexpr (QLDS) {
+#pragma unroll
+    for (int f = 0; f < NF; f += NW) {
+      half8_t hi, lo;
+      make_q(f + wave, hi, lo);
+      qs[(f + wave) * (QSPLIT ? 2 : 1)][lane] = hi;
+      if constexpr (QSPLIT) qs[2 * (f + wave) + 1][lane] = lo;
+    }
+    __syncthreads();
+  } else {
+#pragma unroll
+    for (int f = 0; f < NF; ++f) make_q(f, qr[f][0], qr[f][1]);
+  }
+  auto q_frag = [&](int f, int part) -> half8_t {
+    if constexpr (QLDS) return qs[f * (QSPLIT ? 2 : 1) + part][lane];
+    else return qr[f][part];
+  };
+
+  const int ntiles = (t1 + 31) / 32;
+  u32x4 kr[NDB];
+  // lanes 0..31: the K scale of key `lane`; 32..63: the V scale of key lane - 32
+  // (the loaded bits: converting them here would wait for them here)
+  using SBits = typename std::conditional<SDT == SF_F32, uint32_t, uint16_t>::type;
+  const SBits *const sp = (const SBits *)(h ? vs : ks) + base;
+  SBits sbits;
+  auto load_k = [&](int j) {
+    const int8_t *p = kc + (base + min(32 * j + l32, t1 - 1)) * D + 16 * h;
+#pragma unroll
+    for (int i = 0; i < NDB; ++i) kr[i] = *(const u32x4 *)(p + 32 * i);
+    sbits = sp[min(32 * j + l32, t1 - 1)];
+  };
+  // straight into LDS: lane l's 16 bytes land at 16 l of the load's 1 KB
+  auto load_v = [&](int j, uint8_t *dst) {
+#pragma unroll
+    for (int i = 0; i < VC; ++i) {
+      const int ch = lane + 64 * i, r = ch / (D / 16), p = ch % (D / 16) ^ (r & (D / 16 - 1));
+      __builtin_amdgcn_global_load_lds(
+          (__attribute__((address_space(1))) void *)(vc + (base + min(32 * j + r, t1 - 1)) * D + p * 16),
+          (__attribute__((address_space(3))) void *)(dst + 1024 * i), 16, 0, 0);
+    }
+  };
+
+  float m = -INFINITY, lsum = 0.f;  // the row's maximum; this half's share of its sum
+  // The weights P * V scale go to fp16 halves times 2^10 (less where a V scale
+  // would overflow them; powers of two, exact): a weight of 1e-4 at a scale of
+  // 0.02 keeps its low half instead of rounding among fp16's subnormals.
+  float vmul = 1024.f;
+  float16_t O[NDB];
+#pragma unroll
+  for (int d = 0; d < NDB; ++d)
+#pragma unroll
+    for (int e = 0; e < 16; ++e) O[d][e] = 0.f;
+
+  // Loads complete in order: a tile's V is issued before its K and scales, so
+  // whoever has the K codes in registers finds V in LDS.
+  auto tile = [&](int j, uint8_t *vcur, uint8_t *vnext) {
+    const bool masked = 32 * j + 32 > lo;  // (uniform)
+    float sr;
+    if constexpr (SDT == SF_F32) sr = sf_bitcast<float>(sbits);
+    else sr = (float)sf_bitcast<f16>(sbits);
+    float shrink = 1.f;
+    while (__any(h && fabsf(sr) * vmul > 32768.f && vmul > 0x1p-20f)) {
+      vmul *= 0.25f;
+      shrink *= 0.25f;
+    }
+    scl[wave][h][l32] = sr * (h ? vmul : qscale);
+    load_v(j + NW, vnext);
+    __builtin_amdgcn_sched_barrier(0);
+    float16_t S = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int f = 0; f < NF; ++f) {
+      const u32x4 w = kr[f >> 1];
+      const half8_t a = (f & 1) ? i8x8_to_h8(w.z, w.w) : i8x8_to_h8(w.x, w.y);
+      S = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, q_frag(f, 0), S, 0, 0, 0);
+      if constexpr (QSPLIT) S = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, q_frag(f, 1), S, 0, 0, 0);
+      if (f & 1) __builtin_amdgcn_sched_barrier(0);  // (converting further ahead costs registers)
+    }
+    load_k(j + NW);  // (past the last tile: clamped, never used)
+    float sc[16], mx = -INFINITY;
+#pragma unroll
+    for (int e4 = 0; e4 < 4; ++e4) {
+      const float4_t k4 = *(const float4_t *)&scl[wave][0][8 * e4 + 4 * h];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) sc[4 * e4 + i] = S[4 * e4 + i] * k4[i];
+    }
+    const int left = lim - 32 * j - 4 * h;  // the lane's keys e: 8 (e / 4) + e % 4 < left
+    if (masked) {
+#pragma unroll
+      for (int e = 0; e < 16; ++e) sc[e] = 8 * (e >> 2) + (e & 3) < left ? sc[e] : -INFINITY;
+    }
+#pragma unroll
+    for (int e = 0; e < 16; ++e) mx = fmaxf(mx, sc[e]);
+    const float2_t mp = sf_swap32_pair(mx);
+    const float m_new = fmaxf(m, fmaxf(mp.x, mp.y));
+    const float m_ref = m_new == -INFINITY ? 0.f : m_new;
+    if (__any(m_new != m) || shrink != 1.f) {
+      const float cf = __builtin_amdgcn_exp2f(m - m_ref);  // exp2(-inf) = 0
+      lsum *= cf;
+#pragma unroll
+      for (int d = 0; d < NDB; ++d) O[d] *= cf * shrink;
+      m = m_new;
+    }
+    half8_t ph[2], pl[2];
+    float ps = 0.f;
+#pragma unroll
+    for (int e4 = 0; e4 < 4; ++e4) {
+      float4_t v4 = *(const float4_t *)&scl[wave][1][8 * e4 + 4 * h];
+      if (masked) {  // masked keys weigh exactly 0 (their scale may be any value)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v4[i] = 8 * e4 + i < left ? v4[i] : 0.f;
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int e = 4 * e4 + i;
+        const float p = __builtin_amdgcn_exp2f(sc[e] - m_ref);
+        ps += p;
+        // one rounding to fp32 that both halves see (contracted into the fp16
+        // conversion, the high half could differ from the one the low half completes)
+        const float pv = sf_opaque(p * v4[i]);
+        const f16 hi = (f16)pv;
+        ph[e >> 3][e & 7] = hi;
+        pl[e >> 3][e & 7] = (f16)(pv - (float)hi);
+      }
+    }
+    lsum += ps;
+    // V fragment f = 2 db + s: lane (dim 32 db + l32, half h), the eight keys of
+    // slice s. In each group of 16 lanes the even lanes' addresses give the eight
+    // keys at dims 0..7 of the group's 16, the odd lanes' at dims 8..15.
+    const int kk = (lane & 15) >> 1, row = 4 * h + (kk < 4 ? kk : 4 + kk);
+    const uint8_t *vp = vcur + row * D + 8 * (lane & 1);
+    const int sw = row & (D / 16 - 1), p0 = (lane >> 4) & 1;
+#pragma unroll
+    for (int f = 0; f < NF; ++f) {
+      typedef int v2i __attribute__((ext_vector_type(2)));
+      const v2i r = __builtin_amdgcn_ds_read_tr8_b64_v2i32(
+          (__attribute__((address_space(3))) v2i *)(vp + 16 * (f & 1) * D + ((2 * (f >> 1) + p0) ^ sw) * 16));
+      const half8_t a = i8x8_to_h8((uint32_t)r.x, (uint32_t)r.y);
+      O[f >> 1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, ph[f & 1], O[f >> 1], 0, 0, 0);
+      O[f >> 1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, pl[f & 1], O[f >> 1], 0, 0, 0);
+      if (f & 1) __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+
+  if (wave < ntiles) {
+    load_v(wave, v0[wave]);
+    __builtin_amdgcn_sched_barrier(0);
+    load_k(wave);
+#pragma unroll 1
+    for (int j = wave; j < ntiles; j += 2 * NW) {
+      tile(j, v0[wave], v1[wave]);
+      if (j + NW < ntiles) tile(j + NW, v1[wave], v0[wave]);
+    }
+  }
+  const float2_t lp = sf_swap32_pair(lsum);
+  lsum = lp.x + lp.y;
+#pragma unroll
+  for (int d = 0; d < NDB; ++d) O[d] *= 1.f / vmul;
+
+  // ---- merge the wave states pairwise (a wave without tiles holds m = -inf,
+  // l = 0, O = 0): waves 2 and 3 into 0 and 1, then 1 into 0, one 32-dim block
+  // at a time through the V tiles' LDS
+  __builtin_amdgcn_s_waitcnt((15 << 8) | (7 << 4));  // vmcnt(0): no load into LDS is on its way
+#pragma unroll
+  for (int half = NW / 2; half >= 1; half /= 2) {
+    const bool from = wave >= half && wave < 2 * half;
+    float *xs = &scl[0][0][0] + (wave & (half - 1)) * 128, *xo = (float *)v0 + (wave & (half - 1)) * 1024;
+    __syncthreads();  // the tiles, their scales or the last block are read
+    if (from) {
+      xs[lane] = m;
+      xs[64 + lane] = lsum;
+    }
+    float w1 = 0.f, w2 = 0.f;
+#pragma unroll
+    for (int d = 0; d < NDB; ++d) {
+      if (d > 0) __syncthreads();
+      if (from) {
+#pragma unroll
+        for (int e = 0; e < 16; ++e) xo[e * 64 + lane] = O[d][e];
+      }
+      __syncthreads();
+      if (wave >= half) continue;
+      if (d == 0) {
+        const float m2 = xs[lane], l2 = xs[64 + lane];
+        const float M = fmaxf(m, m2), M_ref = M == -INFINITY ? 0.f : M;
+        w1 = __builtin_amdgcn_exp2f(m - M_ref);
+        w2 = __builtin_amdgcn_exp2f(m2 - M_ref);
+        m = M;
+        lsum = fmaf(w2, l2, w1 * lsum);
+      }
+#pragma unroll
+      for (int e = 0; e < 16; ++e) O[d][e] = fmaf(xo[e * 64 + lane], w2, O[d][e] * w1);
+    }
+  }
+  if (wave > 0 || c0 + l32 >= ncol) return;
+  const float inv = lsum > 0.f ? 1.f / lsum : 0.f;
+#pragma unroll
+  for (int d = 0; d < NDB; ++d)
+#pragma unroll
+    for (int e4 = 0; e4 < 4; ++e4) {
+      const size_t o = qrow * D + 32 * d + 8 * e4 + 4 * h;
+      const float4_t v = float4_t{O[d][4 * e4], O[d][4 * e4 + 1], O[d][4 * e4 + 2], O[d][4 * e4 + 3]} * inv;
+      if (odt == SF_F32) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) ((float *)out)[o + i] = v[i];
+      } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          ((uint16_t *)out)[o + i] = odt == SF_BF16 ? sf_f32_to_bf16(v[i]) : sf_bitcast<uint16_t>((f16)v[i]);
+      }
+    }
+}
+
 }  // namespace
 
 // ---------------------------------------------------------------------------
@@ -1331,14 +1617,24 @@ static int prefill_mfma_launch(const char *what, const void *q, int q_dtype, con
              "prefill of %d rows is too long", T_q);
   dim3 grid((unsigned)(nblk * KVH), 1, 1);
   hipStream_t st = (hipStream_t)stream;
+  // 32-row workgroups from one per CU on, 16-row ones below (more of them):
+  // 32 / 8 heads of 128, 128 rows (128 workgroups of 32 rows) 8.3 us against 7.2,
+  // 300 rows (304) 12.0 against 15.2; 14 / 2 heads of 64, 512 rows (224) 9.0
+  // against 8.9, 1000 rows (438) 13.9 against 17.4
+  const long long rblk = (ncol + 31) / 32 * KVH;
+  const bool rows = rblk >= 256;
+  const dim3 rgrid((unsigned)rblk, 1, 1);
 #define SF_PF_LAUNCH(QD, SD, DD)                                                               \
-  k_attn_prefill_mfma<QD, SD, DD><<<grid, kPfWaves * 64, 0, st>>>(                            \
+  if (rows) k_attn_prefill_rows<QD, SD, DD><<<rgrid, 256, 0, st>>>(                            \
+      q, k_codes, k_scales, v_codes, v_scales, out, out_dtype, H, KVH, T_q, T0, T0_dev, T_cap, \
+      qscale);                                                                                 \
+  else k_attn_prefill_mfma<QD, SD, DD><<<grid, kPfWaves * 64, 0, st>>>(                            \
       q, k_codes, k_scales, v_codes, v_scales, out, out_dtype, H, KVH, T_q, T0, T0_dev, T_cap, \
       qscale, vscale)
 #define SF_PF_D(QD, SD)                  \
   do {                                   \
-    if (D == 64) SF_PF_LAUNCH(QD, SD, 64); \
-    else SF_PF_LAUNCH(QD, SD, 128);      \
+    if (D == 64) { SF_PF_LAUNCH(QD, SD, 64); } \
+    else { SF_PF_LAUNCH(QD, SD, 128); }      \
   } while (0)
   if (scale_dtype == SF_F16) {
     if (q_dtype == SF_F32) SF_PF_D(SF_F32, SF_F16);
