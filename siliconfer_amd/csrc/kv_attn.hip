@@ -598,13 +598,32 @@ k_attn_mfma(const void *__restrict__ q, const int8_t *__restrict__ kc, const voi
 #pragma unroll
   for (int d = 0; d < DB; ++d) O[d] = float4_t{0.f, 0.f, 0.f, 0.f};
 
+  // Where a wave runs more than one tile, the weights P * V scale go to fp16
+  // halves times 2^10 (less where a V scale would overflow them; powers of two,
+  // exact), so that small weights keep their low half instead of rounding among
+  // fp16's subnormals (error against 64 bits at four sequences of 8191 tokens in
+  // 16 splits: 5.9e-6 without, 3e-7 with). Short runs do without: it costs a
+  // decode step of one tile a wave 0.1 us a launch.
+  const bool deep = mine > 1;  // (wave-uniform)
+  float vmul = deep ? 1024.f : 1.f;
+
   auto compute = [&](int j, const Tile &tl) {
     const int tb = 32 * j;
-    float tks[8], tvs[8];
+    float tks[8], tvs[8], vmx = 0.f, shrink = 1.f;
 #pragma unroll
     for (int r = 0; r < 8; ++r) {
       tks[r] = scale_of(tl.kw, r);
       tvs[r] = scale_of(tl.vw, r);
+    }
+    if (deep) {
+#pragma unroll
+      for (int r = 0; r < 8; ++r) vmx = fmaxf(vmx, tb + tok_of(r) < Tv ? fabsf(tvs[r]) : 0.f);
+      while (__any(vmx * vmul > 32768.f && vmul > 0x1p-20f)) {
+        vmul *= 0.25f;
+        shrink *= 0.25f;
+      }
+#pragma unroll
+      for (int r = 0; r < 8; ++r) tvs[r] *= vmul;
     }
     // S^T for the two 16-token halves
     float4_t S[2];
@@ -639,7 +658,7 @@ k_attn_mfma(const void *__restrict__ q, const int8_t *__restrict__ kc, const voi
       const float p = __builtin_amdgcn_exp2f(sc[r] - m_ref);
       ps += p;
       // masked tokens weigh exactly 0 (their scale may be any stale value)
-      const float pv = tb + tok_of(r) < Tv ? p * tvs[r] : 0.f;
+      const float pv = sf_opaque(tb + tok_of(r) < Tv ? p * tvs[r] : 0.f);
       ph[r] = (f16)pv;
       pl[r] = (f16)(pv - (float)ph[r]);
     }
@@ -659,7 +678,7 @@ k_attn_mfma(const void *__restrict__ q, const int8_t *__restrict__ kc, const voi
       const v2i r = __builtin_amdgcn_ds_read_tr8_b64_v2i32(
           (__attribute__((address_space(3))) v2i *)(vt + vtok * PITCH + 16 * d + 8 * (hl & 1)));
       const half8_t a = i8x8_to_h8((uint32_t)r.x, (uint32_t)r.y);
-      O[d] *= c;
+      O[d] *= c * shrink;
       O[d] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, ph, O[d], 0, 0, 0);
       O[d] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, pl, O[d], 0, 0, 0);
     }
@@ -678,6 +697,10 @@ k_attn_mfma(const void *__restrict__ q, const int8_t *__restrict__ kc, const voi
     }
   }
   lsum = sum_x16_x32(lsum);
+  if (deep) {
+#pragma unroll
+    for (int d = 0; d < DB; ++d) O[d] *= 1.f / vmul;
+  }
 
   // ---- merge the 4 wave states (LDS)
   float *ms = smem + NW * 32 * PITCH / 4;  // [NW][16]
@@ -1372,6 +1395,13 @@ extern "C" size_t sf_attn_workspace_bytes(int B, int H, int D, int n_splits) {
   return sf_split_ws_parts(B * H, D, n_splits, &acc_off, &ml_off);
 }
 
+// The default split count of one sequence over few kv heads.
+static int splits_by_length(int T) {
+  if (T <= 160) return 1;
+  const int s = (T + (T <= 2048 ? 31 : 63)) / (T <= 2048 ? 32 : 64);
+  return s < 8 ? 8 : s > 128 ? 128 : s;
+}
+
 extern "C" int sf_attn_default_splits_d(int B, int KVH, int T, int D) {
   // One split (one workgroup per (b, kv head), no merge launch) up to 160
   // tokens; beyond, 32 tokens per split up to 2048 cached tokens and 64 above,
@@ -1385,14 +1415,24 @@ extern "C" int sf_attn_default_splits_d(int B, int KVH, int T, int D) {
   //                 (128; 64: 10.1).
   // Eight waves per split workgroup (one tile each) instead of four measured
   // no faster at 4096-16384 tokens.
-  (void)B;
-  (void)KVH;
+  // Where that is more than one workgroup a CU (several sequences or many kv
+  // heads), only as many splits as bring one, or up to two with 128 tokens each
+  // (a tile for each of the workgroup's four waves): more add workgroups that
+  // wait their turn and partials to merge. Four sequences at 32 / 8 heads of 128
+  // (us; the count before in parentheses): T = 400: 7.7 (8.2); 1000: 9.2 (13.3);
+  // 2000: 11.4 (22.4); 4096: 14.7 (24.2); 8191: 22.4 (42.8). One sequence there:
+  // 2000: 7.8 (8.4); 8191: 11.9 (15.8); 16384: 14.9 (17.4). Four at 32 / 32 heads:
+  // 2000: 19.2 (63.2).
   (void)D;
-  if (T <= 160) return 1;
-  const int tps = T <= 2048 ? 32 : 64;
-  int s = (T + tps - 1) / tps;
-  if (s < 8) s = 8;
-  if (s > 128) s = 128;
+  int s = splits_by_length(T);
+  const long long heads = (long long)B * KVH;
+  if (s > 1 && heads > 0 && heads * s > 256) {
+    const int one = (int)((256 + heads - 1) / heads), two = (int)(512 / heads);
+    int t = (T + 127) / 128;
+    if (t > two) t = two;
+    if (t < one) t = one;
+    if (s > t) s = t;
+  }
   return s;
 }
 
@@ -1738,13 +1778,16 @@ extern "C" int sf_attn_decode_i8kv_noalloc(const void *q, int q_dtype, const int
                                            int D, float scale, int n_splits, void *stream) {
   SF_REQUIRE(B > 0 && H > 0 && KVH > 0 && D > 0 && T >= 0 && T <= T_cap, SF_EINVAL,
              "invalid attention shape B=%d H=%d KVH=%d T=%d T_cap=%d D=%d", B, H, KVH, T, T_cap, D);
-  int s = n_splits > 0 ? n_splits : sf_attn_default_splits_d(B, KVH, T, D);
+  // sized by the length alone: the default may split fewer ways, but which
+  // shapes this call takes does not depend on that
+  int s = n_splits > 0 ? n_splits : splits_by_length(T);
   s = s < (T > 0 ? T : 1) ? s : (T > 0 ? T : 1);
   const size_t need = sf_attn_workspace_bytes(B, H, D, s);
   SF_REQUIRE(need <= kNoAllocScratchBytes, SF_EINVAL,
              "sf_attn_decode_i8kv_noalloc: B=%d H=%d D=%d with %d splits needs %zu bytes of "
              "scratch, more than its fixed %zu; use sf_attn_decode_i8kv with a workspace",
              B, H, D, s, need, kNoAllocScratchBytes);
+  if (n_splits <= 0) s = sf_attn_default_splits_d(B, KVH, T, D);
   void *ws = nullptr;
   int rc = scratch_for_current_device(&ws);
   if (rc) return rc;
