@@ -71,8 +71,9 @@ def attention_decode(q: torch.Tensor, k_codes: torch.Tensor, k_scales: torch.Ten
         raise ValueError(f"head_dim={D} exceeds kernel's compile-time max {_MAX_HEAD_DIM}")
     if T is None:
         T = T_cap
-    ks = k_scales.reshape(B, KVH, T_cap)
-    vs = v_scales.reshape(B, KVH, T_cap)
+    rows = (B, KVH, T_cap)
+    ks = k_scales if k_scales.shape == rows else k_scales.reshape(rows)
+    vs = v_scales if v_scales.shape == rows else v_scales.reshape(rows)
     if ks.dtype != vs.dtype or ks.dtype not in (torch.float16, torch.float32):
         raise SFError("k/v scales must both be float16 or both float32")
     if k_codes.dtype != torch.int8 or v_codes.dtype != torch.int8:
@@ -97,7 +98,8 @@ def attention_decode(q: torch.Tensor, k_codes: torch.Tensor, k_scales: torch.Ten
                                  v_codes.data_ptr(), vs.data_ptr(), _lib.dt(ks), out.data_ptr(),
                                  _lib.dt(out), ws.data_ptr(), ws.numel(), B, H, KVH, T, T_cap, D,
                                  float(scale), n_splits, st)
-    _lib.check(rc, "sf_attn_decode_i8kv")
+    if rc:
+        _lib.check(rc, "sf_attn_decode_i8kv")
     return out
 
 

@@ -96,26 +96,26 @@ class Q4Weight:
                out_f32: torch.Tensor | None = None) -> torch.Tensor:
         """x [M, K] (fp16 / bf16 / fp32, on the device) -> [M, N] of out_dtype (default x.dtype)."""
         _lib.require_device(x, "x")
-        if x.dim() != 2 or x.shape[1] != self.in_features:
+        N, K, g = self.out_features, self.in_features, self.group_size
+        if x.dim() != 2 or x.shape[1] != K:
             raise SFError("X/W in_features mismatch")
         M = x.shape[0]
-        N, K, g = self.out_features, self.in_features, self.group_size
-        if out_dtype is None:
-            out_dtype = x.dtype
         if out is None and out_f32 is None:
-            out = torch.empty((M, N), dtype=out_dtype, device=x.device)
+            out = torch.empty((M, N), dtype=out_dtype or x.dtype, device=x.device)
         if M == 0:
             return out if out is not None else out_f32
+        xdt = _lib.dt(x)
+        ydt = _lib.dt(out) if out is not None else _lib.SF_F32
+        bptr, bdt = None, 0
         if bias is not None:
             _lib.require_device(bias, "bias")
+            bptr, bdt = bias.data_ptr(), _lib.dt(bias)
         lib = _lib.load()
-        st = _lib.stream(x)
-        ydt = _lib.dt(out) if out is not None else _lib.SF_F32
-        bdt = _lib.dt(bias) if bias is not None else 0
-        ws_bytes = lib.sf_q4_matmul_workspace_bytes(M, N, K, g, _lib.dt(x))
+        ws_bytes = lib.sf_q4_matmul_workspace_bytes(M, N, K, g, xdt)
         ws = torch.empty(ws_bytes, dtype=torch.uint8, device=x.device) if ws_bytes else None
-        rc = lib.sf_q4_matmul(self.blob.data_ptr(), x.data_ptr(), _lib.dt(x), _lib.ptr(out), ydt,
-                              _lib.ptr(out_f32), _lib.ptr(bias), bdt, M, N, K, g,
-                              int(self.has_zeros), _lib.ptr(ws), ws_bytes, st)
-        _lib.check(rc, "sf_q4_matmul")
+        rc = lib.sf_q4_matmul(self.blob.data_ptr(), x.data_ptr(), xdt, _lib.ptr(out), ydt,
+                              _lib.ptr(out_f32), bptr, bdt, M, N, K, g, int(self.has_zeros),
+                              _lib.ptr(ws), ws_bytes, _lib.stream(x))
+        if rc:
+            _lib.check(rc, "sf_q4_matmul")
         return out if out is not None else out_f32

@@ -21,6 +21,8 @@ import torch
 
 from ..kernels.q4 import Q4Weight
 
+_ACT_DTYPES = (torch.float16, torch.bfloat16, torch.float32)
+
 
 class Q4Linear(torch.nn.Module):
     """Holds `_packed` uint8 [out, in/2], `_scales` [out, n_groups], `_zeros`
@@ -48,14 +50,14 @@ class Q4Linear(torch.nn.Module):
         return self.weight.device
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        orig = x.shape
-        x2 = x.reshape(-1, self.in_features)
+        rows = x.dim() == 2 and x.shape[1] == self.in_features
+        x2 = x if rows else x.reshape(-1, self.in_features)
         if not x2.is_contiguous():
             x2 = x2.contiguous()
-        if x2.dtype not in (torch.float16, torch.bfloat16, torch.float32):
+        if x2.dtype not in _ACT_DTYPES:
             x2 = x2.float()
         y = self.weight.matmul(x2, out_dtype=torch.float32, bias=self.bias)
-        return y.reshape(*orig[:-1], self.out_features)
+        return y if rows else y.reshape(*x.shape[:-1], self.out_features)
 
     __call__ = torch.nn.Module.__call__
 
