@@ -168,6 +168,25 @@ int sf_q4_matmul(const void *blob, const void *x, int x_dtype, void *y, int y_dt
                  const void *bias, int bias_dtype, int M, int N, int K, int group_size,
                  int has_zeros, void *workspace, size_t workspace_bytes, void *stream);
 
+/* Several weights of one in_features, group size and zero-point form on the
+ * same X in one launch (1 to 3 of them; more than 16 rows):
+ *   op SF_GROUP_CONCAT: Y[M][sum N] = their outputs side by side, biases[i]
+ *     (NULL: none; biases may be NULL itself) of bias_dtypes[i] added;
+ *   op SF_GROUP_SWIGLU: Y[M][I] = silu(X . gate^T) * (X . up^T), sf_silu_mul of
+ *     the two projections; blobs gate, up of N = I each, or one of N = 2 I
+ *     holding gate's rows, then up's. No biases.
+ * sf_q4_matmul_group_supported: 1 and the workspace size (16-byte aligned, may
+ * be 0 -> NULL ok) where the call runs such a shape, else 0 (run the weights
+ * one by one). */
+#define SF_GROUP_CONCAT 0
+#define SF_GROUP_SWIGLU 1
+int sf_q4_matmul_group_supported(int op, int n, const int *Ns, int M, int K, int group_size,
+                                 int x_dtype, size_t *workspace_bytes);
+int sf_q4_matmul_group(int op, int n, const void *const *blobs, const int *Ns,
+                       const void *const *biases, const int *bias_dtypes, const void *x,
+                       int x_dtype, void *y, int y_dtype, int M, int K, int group_size,
+                       int has_zeros, void *workspace, size_t workspace_bytes, void *stream);
+
 /* The prefill GEMM with its K-split partials left for the next op (no
  * counterpart in the reference, whose q4_gemm returns Y; here the decoder's
  * prompt path folds the residual delta into the RMSNorm that follows).

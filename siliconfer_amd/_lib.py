@@ -21,6 +21,7 @@ LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "libsiliconf
 
 SF_F32, SF_F16, SF_BF16 = 0, 1, 2
 SF_PRE_RMSNORM, SF_PRE_SILU_MUL = 1, 2
+SF_GROUP_CONCAT, SF_GROUP_SWIGLU = 0, 1
 SF_CHAIN_IN_X0, SF_CHAIN_IN_PREV, SF_CHAIN_IN_SWIGLU = 0, 1, 2
 SF_CHAIN_MAX_PHASES = 8
 _DT = {torch.float32: SF_F32, torch.float16: SF_F16, torch.bfloat16: SF_BF16}
@@ -53,6 +54,9 @@ _SIGS = {
     "sf_q4_matmul_workspace_bytes": (_c_sz, [_c_i, _c_i, _c_i, _c_i, _c_i]),
     "sf_q4_matmul": (_c_i, [_c_p, _c_p, _c_i, _c_p, _c_i, _c_p, _c_p, _c_i,
                             _c_i, _c_i, _c_i, _c_i, _c_i, _c_p, _c_sz, _c_p]),
+    "sf_q4_matmul_group_supported": (_c_i, [_c_i, _c_i, _c_p, _c_i, _c_i, _c_i, _c_i, _c_p]),
+    "sf_q4_matmul_group": (_c_i, [_c_i, _c_i, _c_p, _c_p, _c_p, _c_p, _c_p, _c_i, _c_p, _c_i, _c_i,
+                                  _c_i, _c_i, _c_i, _c_p, _c_sz, _c_p]),
     "sf_q4_gemm_splits": (_c_i, [_c_i, _c_i, _c_i, _c_i]),
     "sf_q4_gemm_partials": (_c_i, [_c_p, _c_p, _c_i, _c_i, _c_i, _c_i, _c_i, _c_i, _c_p, _c_sz,
                                    _c_p]),

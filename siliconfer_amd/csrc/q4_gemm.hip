@@ -22,15 +22,19 @@
 // When the tile grid is too small to fill the GPU, K is split across
 // workgroups into an fp32 workspace and summed by a second kernel in a fixed
 // order.
+#include <limits.h>
 #include <math.h>
 
 #include "q4_gemm_rows.h"
 #include "q4_gemv_blk.h"
 #include "sf_common.h"
 
-bool sf_gemm_rows_f16(const sf_gemm::RowsArgs &a, bool asym, int rb, int kw, hipStream_t s);
-bool sf_gemm_rows_bf16(const sf_gemm::RowsArgs &a, bool asym, int rb, int kw, hipStream_t s);
-bool sf_gemm_rows_f32(const sf_gemm::RowsArgs &a, bool asym, int rb, int kw, hipStream_t s);
+bool sf_gemm_rows_f16(const sf_gemm::RowsArgs &a, const sf_gemm::RowsGroupArgs *group, bool asym, int rb, int kw,
+                      hipStream_t s);
+bool sf_gemm_rows_bf16(const sf_gemm::RowsArgs &a, const sf_gemm::RowsGroupArgs *group, bool asym, int rb, int kw,
+                      hipStream_t s);
+bool sf_gemm_rows_f32(const sf_gemm::RowsArgs &a, const sf_gemm::RowsGroupArgs *group, bool asym, int rb, int kw,
+                      hipStream_t s);
 
 namespace {
 
@@ -463,6 +467,13 @@ k_split_f32(const float *__restrict__ x, uint16_t *__restrict__ hi, uint16_t *__
   ((u32x4 *)lo)[t] = l;
 }
 
+const void *split_rows(const float *x, void *halves, int M, int K, hipStream_t s) {
+  uint16_t *xs = (uint16_t *)halves;
+  const size_t n = (size_t)M * K;
+  k_split_f32<<<(unsigned)((n / 8 + 255) / 256), 256, 0, s>>>(x, xs, xs + n, n / 8);
+  return xs;
+}
+
 // K split count: enough (tile, split) workgroups to give every CU one, each
 // split keeping at least 4 K steps.
 int choose_ksplit(int M, int N, int K) {
@@ -507,10 +518,29 @@ void rows_tile(int M, int N, int K, int xdt, int ks, int *rb, int *kw) {
   }
 }
 
-int rows_run(const sf_gemm::RowsArgs &a, int xdt, bool asym, int rb, int kw, hipStream_t s) {
-  const bool built = xdt == SF_F32   ? sf_gemm_rows_f32(a, asym, rb, kw, s)
-                     : xdt == SF_F16 ? sf_gemm_rows_f16(a, asym, rb, kw, s)
-                                     : sf_gemm_rows_bf16(a, asym, rb, kw, s);
+// A weight as a RowsSeg whose columns begin at output column `col`.
+sf_gemm::RowsSeg rows_seg(const void *blob, const void *bias, int bdt, int N, int K, int g, bool asym,
+                          int tile, int col) {
+  BlobLayout L;
+  sf_blob_layout(N, K, g, asym, &L);
+  const uint8_t *w = (const uint8_t *)blob;
+  return {w, (const f16 *)(w + L.s_off), asym ? w + L.z_off : nullptr, bias, bdt, N, 0, tile, col};
+}
+
+constexpr sf_gemm::RowsSeg kNoSeg = {nullptr, nullptr, nullptr, nullptr, 0, 0, 0, INT_MAX, 0};
+
+sf_gemm::RowsArgs rows_args(const void *blob, const void *x, void *y, float *y32, const void *bias, float *part,
+                            int ydt, int bdt, int M, int N, int K, int g, bool asym, int ks, bool vec) {
+  const int pairs = (K + 127) / 128;
+  return {rows_seg(blob, bias, bdt, N, K, g, asym, 0, 0), x, y, y32, part, ydt, M, K, N,
+          K / g, g, ks, (pairs + ks - 1) / ks, (N + 127) / 128, vec};
+}
+
+int rows_run(const sf_gemm::RowsArgs &a, int xdt, bool asym, int rb, int kw, hipStream_t s,
+             const sf_gemm::RowsGroupArgs *group = nullptr) {
+  const bool built = xdt == SF_F32   ? sf_gemm_rows_f32(a, group, asym, rb, kw, s)
+                     : xdt == SF_F16 ? sf_gemm_rows_f16(a, group, asym, rb, kw, s)
+                                     : sf_gemm_rows_bf16(a, group, asym, rb, kw, s);
   return built ? SF_OK : sf_fail(SF_EUNSUPPORTED, "no GEMM tile of %d row blocks, %d K groups", rb, kw);
 }
 
@@ -661,9 +691,8 @@ static int q4_gemm_impl(const void *blob, const void *x, int x_dtype, void *y, i
   if (x_dtype != SF_F32 && rows_takes(M, K, group_size, x_dtype)) {
     int rb, kw;
     rows_tile(M, N, K, x_dtype, ksplit, &rb, &kw);
-    const int pairs = (K + 127) / 128;
-    const int rr = rows_run({w, st, zt, x, y, y_f32, bias, part, y_dtype, bias_dtype, M, N, K, L.G,
-                             group_size, ksplit, (pairs + ksplit - 1) / ksplit, vec},
+    const int rr = rows_run(rows_args(blob, x, y, y_f32, bias, part, y_dtype, bias_dtype, M, N, K, group_size,
+                                      has_zeros, ksplit, vec),
                             x_dtype, has_zeros, rb, kw, s);
     if (rr) return rr;
   } else {
@@ -757,24 +786,98 @@ extern "C" int sf_q4_matmul(const void *blob, const void *x, int x_dtype, void *
              "matmul workspace too small: %zu < %zu", workspace_bytes, p.bytes);
   SF_REQUIRE(p.bytes == 0 || ((uintptr_t)workspace & 15) == 0, SF_EINVAL,
              "matmul workspace must be 16-byte aligned");
-  BlobLayout L;
-  sf_blob_layout(N, K, group_size, has_zeros, &L);
-  const uint8_t *w = (const uint8_t *)blob;
   hipStream_t s = (hipStream_t)stream;
-  if (x_dtype == SF_F32) {
-    uint16_t *xs = (uint16_t *)((char *)workspace + p.parts);
-    const size_t n = (size_t)M * K;
-    k_split_f32<<<(unsigned)((n / 8 + 255) / 256), 256, 0, s>>>((const float *)x, xs, xs + n, n / 8);
-    x = xs;
-  }
-  const int pairs = (K + 127) / 128;
+  if (x_dtype == SF_F32) x = split_rows((const float *)x, (char *)workspace + p.parts, M, K, s);
   const bool vec = N % 8 == 0 && ((uintptr_t)y & 15) == 0 && ((uintptr_t)y_f32 & 15) == 0;
-  const int rr = rows_run({w, (const f16 *)(w + L.s_off), has_zeros ? w + L.z_off : nullptr, x, y, y_f32,
-                           bias, (float *)workspace, y_dtype, bias_dtype, M, N, K, L.G, group_size, p.ks,
-                           (pairs + p.ks - 1) / p.ks, vec},
+  const int rr = rows_run(rows_args(blob, x, y, y_f32, bias, (float *)workspace, y_dtype, bias_dtype, M, N, K,
+                                    group_size, has_zeros, p.ks, vec),
                           x_dtype, has_zeros, p.rb, p.kw, s);
   if (rr) return rr;
   const int rc = sf_check_launch("sf_q4_matmul");
   if (rc || p.ks == 1) return rc;
   return splitk_reduce((const float *)workspace, y, y_dtype, y_f32, bias, bias_dtype, M, N, p.ks, vec, s);
+}
+
+// One k_q4_gemm_rows launch for several weights on the same rows. Taken where
+// every weight by itself goes to the rows kernel and together they need no K
+// split (a split's partials have one weight's layout); else the caller runs
+// them one by one.
+static bool group_plan(int op, int n, const int *Ns, int M, int K, int g, int xdt, MatmulPlan *p, int *tiles) {
+  if (n < 1 || n > 3 || !Ns || M <= kGemmGemvRows || K <= 0 || g <= 0 || K % g || !rows_takes(M, K, g, xdt))
+    return false;
+  if (op == SF_GROUP_SWIGLU && (n > 2 || (n == 1 ? Ns[0] % 2 : Ns[0] != Ns[1]))) return false;
+  long long t = 0, cols = 0;
+  for (int i = 0; i < n; ++i) {
+    if (Ns[i] <= 0) return false;
+    t += (Ns[i] + 127) / 128;
+    cols += Ns[i];
+  }
+  if (op == SF_GROUP_SWIGLU) t = (cols / 2 + 63) / 64;
+  if (t > (1 << 20) || cols > INT_MAX) return false;
+  *tiles = (int)t;
+  matmul_plan(M, *tiles * 128, K, g, false, xdt, false, p);
+  return p->route == MatmulPlan::ROWS && p->ks == 1;
+}
+
+extern "C" int sf_q4_matmul_group_supported(int op, int n, const int *Ns, int M, int K, int group_size,
+                                            int x_dtype, size_t *workspace_bytes) {
+  MatmulPlan p;
+  int tiles;
+  if (op != SF_GROUP_CONCAT && op != SF_GROUP_SWIGLU) return 0;
+  if (x_dtype != SF_F16 && x_dtype != SF_BF16 && x_dtype != SF_F32) return 0;
+  if (!group_plan(op, n, Ns, M, K, group_size, x_dtype, &p, &tiles)) return 0;
+  if (workspace_bytes) *workspace_bytes = p.bytes;
+  return 1;
+}
+
+extern "C" int sf_q4_matmul_group(int op, int n, const void *const *blobs, const int *Ns,
+                                  const void *const *biases, const int *bias_dtypes, const void *x,
+                                  int x_dtype, void *y, int y_dtype, int M, int K, int group_size,
+                                  int has_zeros, void *workspace, size_t workspace_bytes, void *stream) {
+  size_t need = 0;
+  SF_REQUIRE(blobs && Ns && sf_q4_matmul_group_supported(op, n, Ns, M, K, group_size, x_dtype, &need),
+             SF_EUNSUPPORTED, "no grouped launch for op=%d n=%d M=%d K=%d group_size=%d", op, n, M, K, group_size);
+  SF_REQUIRE(op == SF_GROUP_CONCAT || !biases, SF_EUNSUPPORTED, "the SwiGLU form takes no biases");
+  SF_REQUIRE(!biases || bias_dtypes, SF_EINVAL, "null pointer argument");
+  int width = 0;
+  for (int i = 0; i < n; ++i) {
+    const void *bias = biases ? biases[i] : nullptr;
+    const int bad = gemm_check(blobs[i], x, x_dtype, y, y_dtype, nullptr, bias, bias ? bias_dtypes[i] : 0, M,
+                               Ns[i], K, group_size);
+    if (bad) return bad;
+    width += Ns[i];
+  }
+  SF_REQUIRE(need == 0 || (workspace && workspace_bytes >= need && ((uintptr_t)workspace & 15) == 0), SF_EINVAL,
+             "matmul workspace too small or not 16-byte aligned: %zu < %zu", workspace_bytes, need);
+  MatmulPlan p;
+  int tiles;
+  group_plan(op, n, Ns, M, K, group_size, x_dtype, &p, &tiles);
+  hipStream_t s = (hipStream_t)stream;
+  if (x_dtype == SF_F32) x = split_rows((const float *)x, workspace, M, K, s);
+  sf_gemm::RowsGroupArgs a{rows_args(blobs[0], x, y, nullptr, nullptr, nullptr, y_dtype, 0, M, Ns[0], K, group_size,
+                                     has_zeros, 1, true),
+                           {kNoSeg, kNoSeg},
+                           false};
+  a.tiles = tiles;
+  if (op == SF_GROUP_SWIGLU) {
+    const int I = n == 1 ? Ns[0] / 2 : Ns[0];
+    a.swiglu = true;
+    a.ld = I;
+    a.more[0] = n == 1 ? a.seg : rows_seg(blobs[1], nullptr, 0, I, K, group_size, has_zeros, 0, 0);
+    a.seg.N = a.more[0].N = I;
+    a.more[0].n_off = n == 1 ? I : 0;
+  } else {
+    a.ld = width;
+    int tile = 0, col = 0;
+    for (int i = 0; i < n; ++i) {
+      (i ? a.more[i - 1] : a.seg) = rows_seg(blobs[i], biases ? biases[i] : nullptr, bias_dtypes && biases ? bias_dtypes[i] : 0,
+                          Ns[i], K, group_size, has_zeros, tile, col);
+      tile += (Ns[i] + 127) / 128;
+      col += Ns[i];
+      a.vec = a.vec && Ns[i] % 8 == 0;
+    }
+  }
+  a.vec = a.vec && a.ld % 8 == 0 && ((uintptr_t)y & 15) == 0;
+  const int rr = rows_run(a, x_dtype, has_zeros, p.rb, p.kw, s, &a);
+  return rr ? rr : sf_check_launch("sf_q4_matmul_group");
 }

@@ -3,6 +3,7 @@
 #pragma once
 
 #include <atomic>
+#include <type_traits>
 
 #include "q4_gemv_blk.h"
 #include "sf_common.h"
@@ -20,17 +21,30 @@ typedef __attribute__((address_space(3))) void lds_void;
 // Wait for this wave's LDS operations (vm and exp left at their maxima).
 #define SF_WAIT_LGKM0() __builtin_amdgcn_s_waitcnt(15 | (3 << 14) | (7 << 4))
 
-struct RowsArgs {
+// One weight of a call (n_off: its first row inside the blob).
+struct RowsSeg {
   const uint8_t *wq;   // blob: codes
   const f16 *st;       // scales
   const uint8_t *zt;   // zero-points (asymmetric)
+  const void *bias;
+  int bdt, N, n_off, tile, col;  // tile: its first column tile; col: its first output column
+};
+
+struct RowsArgs {
+  RowsSeg seg;
   const void *x;       // activations [M][K] (fp32: the bf16 high rows, then the low rows)
   void *y;
   float *y32;
-  const void *bias;
   float *part;
-  int ydt, bdt, M, N, K, G, g, ksplit, pairs_per_split;
+  int ydt, M, K, ld, G, g, ksplit, pairs_per_split, tiles;  // ld: outputs a row
   bool vec;
+};
+
+// Several weights (unused: tile past every column tile), or swiglu: seg gate,
+// more[0] up, y = silu(gate) * up. A single weight's kernel is not passed these.
+struct RowsGroupArgs : RowsArgs {
+  RowsSeg more[2];
+  bool swiglu;
 };
 
 // One output value's bias.
@@ -156,6 +170,12 @@ constexpr int rows_lds_bytes() {
 //    group (y = sum_g s_g sum_k x_k (q_k - z)), one row block behind its MFMAs.
 //    fp32 activations: X holds bf16 high rows, then low rows; two MFMAs an
 //    operand.
+//  * Up to three weights a launch on the same rows (q|k|v): column tiles of each,
+//    side by side in one output. A small weight's tiles fill the last round of
+//    a large one's, the rows are split into halves once and nothing
+//    concatenates afterwards: the 8B attention layer over 1500 rows 415 -> 350 us,
+//    its MLP over 333 rows 318 -> 297 (fp32 both). swiglu: waves 0, 1 take 64 gate columns and waves
+//    2, 3 the same columns of up, and the output tile is silu(gate) * up.
 //  * KW = 2: a second set of four waves takes the other half of the K steps and
 //    the sums meet in LDS (two waves a SIMD without a second output tile).
 // The kernel it replaced staged converted codes through LDS with separate
@@ -171,9 +191,9 @@ constexpr int rows_lds_bytes() {
 // blocks (one wave a SIMD: 234), slot rings of eight with four code sets and a
 // pinned MFMA / VALU interleave (4% slower over the sweep), 256 columns a
 // workgroup (the same).
-template <int XM, bool ASYM, int GK, int RB, int KW>
+template <int XM, bool ASYM, int GK, int RB, int KW, bool GRP>
 __global__ void __launch_bounds__(256 * KW, KW == 1 ? 2 : 1)
-k_q4_gemm_rows(const RowsArgs a) {
+k_q4_gemm_rows(const std::conditional_t<GRP, RowsGroupArgs, RowsArgs> a) {
   constexpr bool SPLIT = XM == SF_F32, F16 = XM == SF_F16;
   constexpr int NF = RB * (SPLIT ? 2 : 1);  // 32-row blocks in LDS
   constexpr int STAGE = NF * 32 * 128;
@@ -186,9 +206,26 @@ k_q4_gemm_rows(const RowsArgs a) {
   const int kg = KW == 1 ? 0 : __builtin_amdgcn_readfirstlane(tid >> 8);  // its K group
   uint8_t *const smem = lds + kg * R_SLOTS * STAGE;
   const int l32 = lane & 31, h = lane >> 5;
-  const int m0 = blockIdx.y * (32 * RB), n0 = blockIdx.x * R_BN;
+  const int m0 = blockIdx.y * (32 * RB), bx = blockIdx.x;
   const int split = blockIdx.z;
-  const int M = a.M, N = a.N, K = a.K, G = a.G;
+  const int M = a.M, K = a.K, G = a.G;
+  // The wave's weight (one for the workgroup but for swiglu). Every candidate is
+  // read with the other arguments and selected: an indexed argument would be a
+  // second memory round trip in front of the first load (512 rows on 4864 x 896
+  // 12.9 us against 12.2, and 37 rows on 11008 x 4096 16.3 against 15.8; 15.6
+  // with one weight's arguments only, so that has its own code).
+  RowsSeg sg = a.seg;
+  bool swiglu = false;
+  if constexpr (GRP) {
+    swiglu = a.swiglu;
+    const bool s1st = swiglu ? wave >= 2 : bx >= a.more[0].tile, s2nd = !swiglu && bx >= a.more[1].tile;
+#define SF_SEG(f) sg.f = s2nd ? a.more[1].f : s1st ? a.more[0].f : sg.f
+    SF_SEG(wq); SF_SEG(st); SF_SEG(zt); SF_SEG(bias); SF_SEG(bdt); SF_SEG(N); SF_SEG(n_off); SF_SEG(tile); SF_SEG(col);
+#undef SF_SEG
+  } else {
+    sg.n_off = sg.tile = sg.col = 0;
+  }
+  const int N = sg.N;
   const int nblk = (K + 127) >> 7;
   // this wave's K steps [s0, s1): the split's pairs dealt to the K groups in
   // contiguous runs; every group runs nst steps (those past s1 add zeros)
@@ -227,10 +264,11 @@ k_q4_gemm_rows(const RowsArgs a) {
   };
 
   // ---- B: the lane's column; a pair of steps is one unit (128 k)
-  const int n = min(n0 + 32 * wave + l32, N - 1);
-  const uint8_t *wp = a.wq + (size_t)(n >> 4) * nblk * 1024 + (h * 16 + (n & 15)) * 16;
-  const f16 *sp = a.st + (size_t)(n >> 3) * G * 8 + (n & 7);
-  const uint8_t *zp = ASYM ? a.zt + (size_t)(n >> 3) * G * 4 + ((n & 7) >> 1) : nullptr;
+  const int wc = swiglu ? 64 * bx + 32 * (wave & 1) : R_BN * (bx - sg.tile) + 32 * wave;
+  const int n = min(wc + l32, N - 1) + sg.n_off;
+  const uint8_t *wp = sg.wq + (size_t)(n >> 4) * nblk * 1024 + (h * 16 + (n & 15)) * 16;
+  const f16 *sp = sg.st + (size_t)(n >> 3) * G * 8 + (n & 7);
+  const uint8_t *zp = ASYM ? sg.zt + (size_t)(n >> 3) * G * 4 + ((n & 7) >> 1) : nullptr;
   const int zsh = 4 * (n & 1);
   struct Pair {
     u32x4 lo, hi;
@@ -400,15 +438,15 @@ k_q4_gemm_rows(const RowsArgs a) {
 
   // ---- output, one 32-row block at a time through LDS (two blocks in turn):
   // whole 128-column row segments, 8 columns a thread
-  const int cl = (tid & 15) * 8, col = n0 + cl, nv = min(8, N - col);
+  const int n0 = R_BN * (bx - sg.tile), cl = (tid & 15) * 8, col = n0 + cl, nv = min(8, N - col);
   float *y32 = a.y32;
   void *y = a.y;
   float bv[8] = {};
   if (a.ksplit > 1) {
-    y32 = a.part + (size_t)split * M * N;
+    y32 = a.part + (size_t)split * M * N;  // one weight: ld = N
     y = nullptr;
-  } else if (a.bias) {
-    for (int e = 0; e < 8; ++e) bv[e] = bias_at(a.bias, a.bdt, min(col + e, N - 1));
+  } else if (!swiglu && sg.bias) {
+    for (int e = 0; e < 8; ++e) bv[e] = bias_at(sg.bias, sg.bdt, min(col + e, N - 1));
   }
 #pragma unroll
   for (int r = 0; r < RB; ++r) {
@@ -419,6 +457,18 @@ k_q4_gemm_rows(const RowsArgs a) {
         ot[(8 * (e >> 2) + 4 * h + (e & 3)) * R_PITCH + 32 * wave + l32] = acc[r][e];
     }
     __syncthreads();
+    if (swiglu) {  // columns 0..63 of the tile: gate, 64..127: up
+      const int rl = tid >> 3, sl = (tid & 7) * 8, sc0 = 64 * bx + sl, sv = min(8, N - sc0);
+      const int row = m0 + 32 * r + rl;
+      if (rl < 32 && row < M && sv > 0) {
+        float v[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+          v[e] = sf_silu_mul(ot[rl * R_PITCH + sl + e], ot[rl * R_PITCH + 64 + sl + e]);
+        store8(v, sv, a.vec, y32, y, a.ydt, (size_t)row * a.ld + sc0);
+      }
+      continue;
+    }
 #pragma unroll
     for (int rl = tid >> 4; rl < 32; rl += 16 * KW) {
       const int row = m0 + 32 * r + rl;
@@ -430,33 +480,34 @@ k_q4_gemm_rows(const RowsArgs a) {
         v[e] = x0[e] + bv[e];
         v[4 + e] = x1[e] + bv[4 + e];
       }
-      if (row < M && nv > 0) store8(v, nv, a.vec, y32, y, a.ydt, (size_t)row * N + col);
+      if (row < M && nv > 0) store8(v, nv, a.vec, y32, y, a.ydt, (size_t)row * (GRP ? a.ld : N) + sg.col + col);
     }
   }
 }
 
-template <int XM, bool ASYM, int GK, int RB, int KW>
-void rows_launch(const RowsArgs &a, hipStream_t s) {
+template <int XM, bool ASYM, int GK, int RB, int KW, bool GRP>
+void rows_launch(const std::conditional_t<GRP, RowsGroupArgs, RowsArgs> &a, hipStream_t s) {
   constexpr int lds = rows_lds_bytes<XM, RB, KW>();
   if constexpr (lds > 64 * 1024) {  // raise the dynamic LDS limit once per variant
     static std::atomic<bool> raised{false};
     if (!raised.load(std::memory_order_acquire)) {
-      (void)hipFuncSetAttribute((const void *)k_q4_gemm_rows<XM, ASYM, GK, RB, KW>,
+      (void)hipFuncSetAttribute((const void *)k_q4_gemm_rows<XM, ASYM, GK, RB, KW, GRP>,
                                 hipFuncAttributeMaxDynamicSharedMemorySize, lds);
       raised.store(true, std::memory_order_release);
     }
   }
-  const dim3 grid((a.N + R_BN - 1) / R_BN, (a.M + 32 * RB - 1) / (32 * RB), a.ksplit);
-  k_q4_gemm_rows<XM, ASYM, GK, RB, KW><<<grid, 256 * KW, lds, s>>>(a);
+  const dim3 grid(a.tiles, (a.M + 32 * RB - 1) / (32 * RB), a.ksplit);
+  k_q4_gemm_rows<XM, ASYM, GK, RB, KW, GRP><<<grid, 256 * KW, lds, s>>>(a);
 }
 
 // The tiles built: rb row blocks of 32 (1..4; fp32 halves up to 2) by kw K
-// groups of waves (1 or 2; two fp32 row blocks 1).
+// groups of waves (1 or 2; two fp32 row blocks 1). group: a itself, if it is one.
 template <int XM>
-bool rows_dispatch(const RowsArgs &a, bool asym, int rb, int kw, hipStream_t s) {
+bool rows_dispatch(const RowsArgs &a, const RowsGroupArgs *group, bool asym, int rb, int kw, hipStream_t s) {
 #define SF_RL(AS, GKV, RBV, KWV)                  \
   if (rb == RBV && kw == KWV) {                   \
-    rows_launch<XM, AS, GKV, RBV, KWV>(a, s);     \
+    if (group) rows_launch<XM, AS, GKV, RBV, KWV, true>(*group, s); \
+    else rows_launch<XM, AS, GKV, RBV, KWV, false>(a, s);        \
     return true;                                  \
   }
 #define SF_RR(AS, GKV)                            \

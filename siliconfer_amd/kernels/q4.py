@@ -11,6 +11,8 @@ reference takes (K % group_size == 0) computes.
 
 from __future__ import annotations
 
+import ctypes
+
 import numpy as np
 import torch
 
@@ -119,3 +121,46 @@ class Q4Weight:
         if rc:
             _lib.check(rc, "sf_q4_matmul")
         return out if out is not None else out_f32
+
+
+def matmul_group(op: int, weights: list[Q4Weight], x: torch.Tensor, biases=None,
+                 out: torch.Tensor | None = None, out_dtype: torch.dtype | None = None,
+                 ws: torch.Tensor | None = None) -> torch.Tensor | None:
+    """Several weights on the rows x [M, K] in one launch (sf_q4_matmul_group):
+    their outputs side by side [M, sum N], or silu(gate) * up [M, I]. None,
+    with nothing launched, where the shape has no such launch (few rows,
+    weights of different forms, or a workspace ws that is too small)."""
+    w0, n = weights[0], len(weights)
+    K, g = w0.in_features, w0.group_size
+    if x.dim() != 2 or x.shape[1] != K or any(
+            (w.in_features, w.group_size, w.has_zeros, w.device) != (K, g, w0.has_zeros, w0.device)
+            for w in weights):
+        return None
+    lib = _lib.load()
+    M, xdt = x.shape[0], _lib.dt(x)
+    Ns = (ctypes.c_int * n)(*(w.out_features for w in weights))
+    need = ctypes.c_size_t()
+    if not lib.sf_q4_matmul_group_supported(op, n, Ns, M, K, g, xdt, ctypes.byref(need)):
+        return None
+    if ws is not None and ws.numel() < need.value:
+        return None
+    _lib.require_device(x, "x")
+    if ws is None and need.value:
+        ws = torch.empty(need.value, dtype=torch.uint8, device=x.device)
+    if out is None:
+        width = sum(Ns)
+        if op == _lib.SF_GROUP_SWIGLU:
+            width //= 2
+        out = torch.empty((M, width), dtype=out_dtype or x.dtype, device=x.device)
+    bias_p = bias_d = None
+    if biases is not None and any(b is not None for b in biases):
+        for b in biases:
+            if b is not None:
+                _lib.require_device(b, "bias")
+        bias_p = (ctypes.c_void_p * n)(*(_lib.ptr(b) for b in biases))
+        bias_d = (ctypes.c_int * n)(*(0 if b is None else _lib.dt(b) for b in biases))
+    blobs = (ctypes.c_void_p * n)(*(w.blob.data_ptr() for w in weights))
+    _lib.check(lib.sf_q4_matmul_group(op, n, blobs, Ns, bias_p, bias_d, x.data_ptr(), xdt, out.data_ptr(),
+                                      _lib.dt(out), M, K, g, int(w0.has_zeros), _lib.ptr(ws),
+                                      need.value, _lib.stream(x)), "sf_q4_matmul_group")
+    return out

@@ -33,7 +33,7 @@ from .. import _lib
 from .._lib import SFError
 from .config import ModelConfig, rope_freqs as _rope_freqs_np
 from .kv_cache import QuantizedKVCache, dequantize_kv
-from .q4_linear import Q4Linear
+from .q4_linear import Q4Linear, project_group
 
 
 def _on_device(x: torch.Tensor) -> None:
@@ -159,11 +159,18 @@ class Attention(torch.nn.Module):
         _on_device(x)  # every route runs on the GPU; none on the host
         B, T, _ = x.shape
         H, KVH, D = self.num_heads, self.num_kv_heads, self.head_dim
-        q = _project(self.q_proj, x)
-        k = _project(self.k_proj, x)
-        v = _project(self.v_proj, x)
-        if isinstance(cache, QuantizedKVCache) and B == 1:
-            out = self._int8_batch1(q, k, v, cache, T, x.device)
+        int8_batch1 = isinstance(cache, QuantizedKVCache) and B == 1
+        qkv = None
+        if int8_batch1:
+            qkv = project_group(_lib.SF_GROUP_CONCAT, (self.q_proj, self.k_proj, self.v_proj), x)
+        if qkv is None:
+            q = _project(self.q_proj, x)
+            k = _project(self.k_proj, x)
+            v = _project(self.v_proj, x)
+        if int8_batch1:
+            if qkv is None:
+                qkv = torch.cat([q.reshape(T, -1), k.reshape(T, -1), v.reshape(T, -1)], dim=1).contiguous()
+            out = self._int8_batch1(qkv, cache, T, x.device)
             return _project(self.o_proj, out.reshape(1, T, H * D)), cache
         q = q.reshape(B, T, H, D).transpose(1, 2)
         k = k.reshape(B, T, KVH, D).transpose(1, 2)
@@ -191,8 +198,8 @@ class Attention(torch.nn.Module):
         a = _sdpa_causal(q, kc, vc, offset, self.scale)
         return _project(self.o_proj, a.transpose(1, 2).reshape(B, T, H * D)), new_cache
 
-    def _int8_batch1(self, q, k, v, cache: QuantizedKVCache, T: int, device) -> torch.Tensor:
-        """RoPE + int8 append in one launch, then decode or causal prefill
+    def _int8_batch1(self, qkv, cache: QuantizedKVCache, T: int, device) -> torch.Tensor:
+        """From q|k|v rows [T, (H + 2 KVH) D]: RoPE + int8 append in one launch, then decode or causal prefill
         attention over the cache in place; returns [T, H, D] fp32."""
         H, KVH, D = self.num_heads, self.num_kv_heads, self.head_dim
         lib = _lib.load()
@@ -201,7 +208,6 @@ class Attention(torch.nn.Module):
         kq, ks, vq, vs = cache.buffers()
         T_cap = kq.shape[2]
         cos_t, sin_t = self._tables(offset + T, device)
-        qkv = torch.cat([q.reshape(T, -1), k.reshape(T, -1), v.reshape(T, -1)], dim=1).contiguous()
         q_rot = torch.empty((T, H, D), dtype=torch.float32, device=device)
         st = _lib.stream(qkv)
         _lib.check(lib.sf_rope_kv_append(qkv.data_ptr(), cos_t.data_ptr(), sin_t.data_ptr(), cos_t.shape[0],
@@ -233,6 +239,9 @@ class MLP(torch.nn.Module):
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         _on_device(x)
+        act = project_group(_lib.SF_GROUP_SWIGLU, (self.gate_proj, self.up_proj), x)
+        if act is not None:
+            return _project(self.down_proj, act.reshape(*x.shape[:-1], act.shape[1]))
         g = _project(self.gate_proj, x)
         u = _project(self.up_proj, x)
         I = g.shape[-1]

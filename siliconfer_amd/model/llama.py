@@ -31,7 +31,7 @@ import torch
 
 from .. import _lib
 from .._lib import SFError
-from ..kernels.q4 import Q4Weight
+from ..kernels.q4 import Q4Weight, matmul_group
 from .config import ModelConfig, rope_tables
 
 _DT = {torch.float32: _lib.SF_F32, torch.float16: _lib.SF_F16, torch.bfloat16: _lib.SF_BF16}
@@ -579,6 +579,7 @@ class LlamaModel:
         # previous projection's output (Dl) to the residual rows itself
         delta = lambda l: None if res or l < 0 else Dl
         parts = 0  # the previous projection's K-split partials still to add (see _gemm_delta)
+        swiglu = False
         for l, L in enumerate(self.layers):
             qparts = 0  # q|k|v left as K-split partials for RoPE + append to sum
             if fq:
@@ -613,13 +614,17 @@ class LlamaModel:
                 self._gemv_fused_rows(L.gate_up, Hb, RMS, L.w_post, GU, None, T)
             else:
                 self._rmsnorm_delta(Hb, delta(l), parts, L.w_post, Xn, T)
-                self._gemm(L.gate_up, Xn, GU, None)
+                swiglu = (self.fuse and not fd and T > GEMM_GEMV_ROWS and matmul_group(
+                    _lib.SF_GROUP_SWIGLU, [L.gate_up], Xn, out=ACT, ws=self._gemm_ws) is not None)
+                if not swiglu:
+                    self._gemm(L.gate_up, Xn, GU, None)
             parts = 0  # consumed: the o projection's partials are in Hb now
             if fd:
                 self._gemv_fused_rows(L.down, GU, SILU, None, Hb, Hb, T)
                 continue
-            self._chk(lib.sf_silu_mul(GU.data_ptr(), ACT.data_ptr(), _DT[ACT.dtype], T, self.I, st),
-                      "sf_silu_mul")
+            if not swiglu:
+                self._chk(lib.sf_silu_mul(GU.data_ptr(), ACT.data_ptr(), _DT[ACT.dtype], T, self.I, st),
+                          "sf_silu_mul")
             parts = 0
             if res:
                 self._gemm(L.down, ACT, Hb, Hb)

@@ -19,7 +19,8 @@ from __future__ import annotations
 import numpy as np
 import torch
 
-from ..kernels.q4 import Q4Weight
+from .._lib import SF_GROUP_SWIGLU
+from ..kernels.q4 import Q4Weight, matmul_group
 
 _ACT_DTYPES = (torch.float16, torch.bfloat16, torch.float32)
 
@@ -51,11 +52,7 @@ class Q4Linear(torch.nn.Module):
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         rows = x.dim() == 2 and x.shape[1] == self.in_features
-        x2 = x if rows else x.reshape(-1, self.in_features)
-        if not x2.is_contiguous():
-            x2 = x2.contiguous()
-        if x2.dtype not in _ACT_DTYPES:
-            x2 = x2.float()
+        x2 = _rows(x if rows else x.reshape(-1, self.in_features))
         y = self.weight.matmul(x2, out_dtype=torch.float32, bias=self.bias)
         return y if rows else y.reshape(*x.shape[:-1], self.out_features)
 
@@ -65,3 +62,32 @@ class Q4Linear(torch.nn.Module):
         return (f"in_features={self.in_features}, out_features={self.out_features}, "
                 f"group_size={self.group_size}, asym={self._zeros is not None}, "
                 f"bias={self.bias is not None}")
+
+
+def _rows(x2: torch.Tensor) -> torch.Tensor:
+    """The rows as the kernels read them: contiguous, in a type they take."""
+    if not x2.is_contiguous():
+        x2 = x2.contiguous()
+    return x2 if x2.dtype in _ACT_DTYPES else x2.float()
+
+
+def _plain(lin) -> bool:
+    """lin(x) is Q4Linear.forward and nothing else: no hook, override or subclass sees the call."""
+    return (type(lin) is Q4Linear and "forward" not in lin.__dict__ and not lin._forward_hooks
+            and not lin._forward_pre_hooks and not lin._backward_hooks and not lin._backward_pre_hooks
+            and not torch.nn.modules.module._has_any_global_hook())
+
+
+def project_group(op: int, lins, x: torch.Tensor) -> torch.Tensor | None:
+    """Projections of the same x [..., in_features] in one launch, fp32: side by
+    side [rows, sum out_features], or silu(first) * second [rows, out_features].
+    None where they run one by one (dense or hooked layers, few rows, weights of
+    different forms)."""
+    K = x.shape[-1]
+    if x.numel() <= 16 * K or not all(_plain(l) and l.in_features == K for l in lins):
+        return None
+    biases = [l.bias for l in lins]
+    if op == SF_GROUP_SWIGLU and any(b is not None for b in biases):
+        return None
+    return matmul_group(op, [l.weight for l in lins], _rows(x.reshape(-1, K)), biases,
+                        out_dtype=torch.float32)
