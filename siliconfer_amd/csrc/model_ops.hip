@@ -107,17 +107,132 @@ k_rmsnorm_parts(float *__restrict__ x, const float *__restrict__ part, int S, si
     store_as(out, odt, r0 + h, sf_opaque(x[r0 + h] * inv * load_as(w, wdt, h)));
 }
 
+// The two kernels above with a row held in one wave's registers: lane l keeps
+// the float4s l + 64 u (u < NU, H <= 256 NU), so x, the delta or its partials
+// and the weight are all loaded at once and nothing is read again behind a
+// barrier. SfRowNorm's order (its lanes add the same float4s in the same order)
+// and the kernels' arithmetic, so the same bits. SRC: 0 no delta, 1 delta, 2
+// partials. Bound by the latency of one round of loads.
+// Measured (us, looping -> this; no delta / delta / four partials): 1 x 896
+// 3.3 / 3.6 / 3.5 -> 2.4 / 2.5 / 2.9, 512 x 896 3.7 / 4.3 / 4.3 -> 2.8 / 3.2 /
+// 3.6, 1 x 4096 7.4 / 9.8 / 8.3 -> 3.7 / 3.9 / 5.5, 2048 x 4096 16.5 / 28.6 /
+// 43.1 -> 9.8 / 17.6 / 35.6 (5.1, 5.7 and 6.6 TB/s, part of it out of cache).
+template <int NU, int SRC>
+__global__ void __launch_bounds__(64)
+k_rmsnorm_wave(float *__restrict__ x, const float *__restrict__ delta, int S, size_t MN,
+               const float *__restrict__ w, void *__restrict__ out, int odt, int H, float eps) {
+  const int lane = threadIdx.x, n4 = H >> 2;
+  const size_t r0 = (size_t)blockIdx.x * H;
+  float4_t *x4 = (float4_t *)(x + r0);
+  const float4_t *d4 = (const float4_t *)(delta + r0);
+  float4_t v[NU], wv[NU];
+  int at[NU];
+#pragma unroll
+  for (int u = 0; u < NU; ++u) {
+    at[u] = min(lane + 64 * u, n4 - 1);
+    v[u] = x4[at[u]];
+  }
+  if constexpr (SRC == 1) {
+    float4_t d[NU];
+#pragma unroll
+    for (int u = 0; u < NU; ++u) d[u] = d4[at[u]];
+#pragma unroll
+    for (int u = 0; u < NU; ++u) wv[u] = ((const float4_t *)w)[at[u]];
+#pragma unroll
+    for (int u = 0; u < NU; ++u) v[u] += d[u];
+  } else if constexpr (SRC == 2) {
+    constexpr int C = 32 / NU;  // partials of a row in flight
+    float4_t d[NU];
+#pragma unroll
+    for (int u = 0; u < NU; ++u) {
+      d[u] = float4_t{0.f, 0.f, 0.f, 0.f};
+      wv[u] = ((const float4_t *)w)[at[u]];
+    }
+    for (int s0 = 0; s0 < S; s0 += C) {
+      float4_t pv[C][NU];
+#pragma unroll
+      for (int j = 0; j < C; ++j)
+        if (s0 + j < S)
+#pragma unroll
+          for (int u = 0; u < NU; ++u) pv[j][u] = ((const float4_t *)(delta + (size_t)(s0 + j) * MN + r0))[at[u]];
+#pragma unroll
+      for (int j = 0; j < C; ++j)
+        if (s0 + j < S)
+#pragma unroll
+          for (int u = 0; u < NU; ++u) d[u] += pv[j][u];
+    }
+#pragma unroll
+    for (int u = 0; u < NU; ++u) v[u] += d[u];
+  } else {
+#pragma unroll
+    for (int u = 0; u < NU; ++u) wv[u] = ((const float4_t *)w)[at[u]];
+  }
+  float ss = 0.f;
+#pragma unroll
+  for (int u = 0; u < NU; ++u) {
+    const float4_t t = lane + 64 * u < n4 ? v[u] : float4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int e = 0; e < 4; ++e) ss = fmaf(t[e], t[e], ss);
+  }
+  ss = sf_wave_sum(ss);
+  const float inv = 1.f / sqrtf(ss / (float)H + eps);
+#pragma unroll
+  for (int u = 0; u < NU; ++u) {
+    const int i = lane + 64 * u;
+    if (i >= n4) continue;
+    if constexpr (SRC != 0) x4[i] = v[u];
+    float o[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) o[e] = sf_opaque(v[u][e] * inv * wv[u][e]);
+    if (odt == SF_F32) {
+      ((float4_t *)((float *)out + r0))[i] = float4_t{o[0], o[1], o[2], o[3]};
+    } else {
+      uint32_t b[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        b[e] = odt == SF_F16 ? sf_bitcast<uint16_t>((f16)o[e]) : sf_f32_to_bf16(o[e]);
+      ((uint2 *)((uint16_t *)out + r0))[i] = uint2{b[0] | b[1] << 16, b[2] | b[3] << 16};
+    }
+  }
+}
+
+// The register kernel where rows are whole float4s of at most 4096 values in
+// aligned fp32 buffers (false: the caller launches the looping kernel).
+template <int SRC>
+bool rmsnorm_wave(float *x, const float *delta, int S, const void *w, int wdt, void *out, int odt, int rows,
+                  int H, float eps, hipStream_t s) {
+  if (H % 4 || H > 4096 || wdt != SF_F32 ||
+      (((uintptr_t)x | (uintptr_t)delta | (uintptr_t)w | (uintptr_t)out) & 15))
+    return false;
+  const size_t MN = (size_t)rows * H;
+  const float *wf = (const float *)w;
+  if (H <= 1024) k_rmsnorm_wave<4, SRC><<<rows, 64, 0, s>>>(x, delta, S, MN, wf, out, odt, H, eps);
+  else if (H <= 2048) k_rmsnorm_wave<8, SRC><<<rows, 64, 0, s>>>(x, delta, S, MN, wf, out, odt, H, eps);
+  else k_rmsnorm_wave<16, SRC><<<rows, 64, 0, s>>>(x, delta, S, MN, wf, out, odt, H, eps);
+  return true;
+}
+
 // ---------------------------------------------------------------------------
+// Heads (waves) a workgroup of the RoPE + append kernels: four, so that
+// thousands of (row, head) pairs are not bound by workgroup launches (us, one a
+// workgroup -> four: 1500 rows of 32/8 heads of 128 18.7 -> 15.2, 512 rows of
+// 14/2 of 64 4.6 -> 4.0; partials 29.9 -> 27.6, 5.4 -> 5.2), one where the pairs
+// are few and each is better on a CU of its own (partials, 8 rows of 14/2:
+// 2.73 against 2.86).
+constexpr int kRopeWaves = 4;
+int rope_waves(int rows, int heads) { return (long long)rows * heads >= 4096 ? kRopeWaves : 1; }
+
 // One wave per (row, head) of the fused q|k|v projection output
 // qkv [rows][(H + 2 KVH) * D]: sf_rope_append_head (rotate-half RoPE with the
 // host-made fp32 cos / sin tables, q to q_out, k and v quantized per (head,
 // token) into the cache at position pos0 + row, batch 1).
-__global__ void __launch_bounds__(64)
+__global__ void __launch_bounds__(64 * kRopeWaves)
 k_rope_kv_append(const float *__restrict__ qkv, SfRopeAppend a, const int *__restrict__ pos_dev,
                  int pos_host) {
-  const int row = blockIdx.x, head = blockIdx.y;
+  const int row = blockIdx.x, head = blockIdx.y * (blockDim.x >> 6) + (threadIdx.x >> 6);
   const int pos = (pos_dev ? *pos_dev : pos_host) + row;
   if (pos < 0 || pos >= a.T_cap || pos >= a.max_pos) return;  // the host keeps positions in range
+  if (head >= a.H + 2 * a.KVH) return;
   const int width = (a.H + 2 * a.KVH) * a.D;
   sf_rope_append_head(a, qkv + (size_t)row * width + (size_t)head * a.D, head, pos, row);
 }
@@ -126,18 +241,21 @@ k_rope_kv_append(const float *__restrict__ qkv, SfRopeAppend a, const int *__res
 // projection plus its bias: each value summed in split order from 0, then the
 // bias added (the GEMM reduce's arithmetic, so the head sees the values the
 // reduce would have stored), staged in LDS for the head.
-__global__ void __launch_bounds__(64)
+__global__ void __launch_bounds__(64 * kRopeWaves)
 k_rope_kv_append_parts(const float *__restrict__ part, int S, size_t MN,
                        const void *__restrict__ bias, int bdt, SfRopeAppend a,
                        const int *__restrict__ pos_dev, int pos_host) {
-  __shared__ float xs[256];
-  const int row = blockIdx.x, head = blockIdx.y;
+  __shared__ float xs4[kRopeWaves][256];
+  const int wave = threadIdx.x >> 6, row = blockIdx.x, head = blockIdx.y * (blockDim.x >> 6) + wave;
+  float *xs = xs4[wave];
   const int pos = (pos_dev ? *pos_dev : pos_host) + row;
   if (pos < 0 || pos >= a.T_cap || pos >= a.max_pos) return;  // the host keeps positions in range
   const int width = (a.H + 2 * a.KVH) * a.D;
   const size_t base = (size_t)row * width + (size_t)head * a.D;
+  const SfRopeCS cs = sf_rope_load_cs(a, pos);
+  const bool in = head < a.H + 2 * a.KVH;
   constexpr int C = 8;  // partials whose loads go out together
-  for (int d = threadIdx.x; d < a.D; d += 64) {
+  for (int d = threadIdx.x & 63; in && d < a.D; d += 64) {
     float v = 0.f;
     for (int s0 = 0; s0 < S; s0 += C) {
       float pv[C];
@@ -152,7 +270,7 @@ k_rope_kv_append_parts(const float *__restrict__ part, int S, size_t MN,
     xs[d] = v;
   }
   __syncthreads();
-  sf_rope_append_head(a, xs, head, pos, row);
+  if (in) sf_rope_append_head(a, xs, head, pos, row, cs);
 }
 
 // ---------------------------------------------------------------------------
@@ -690,7 +808,11 @@ extern "C" int sf_rmsnorm(float *x, const float *delta, const void *w, int w_dty
   SF_REQUIRE(x && w && out, SF_EINVAL, "null pointer argument");
   SF_REQUIRE(w_dtype >= SF_F32 && w_dtype <= SF_BF16 && out_dtype >= SF_F32 && out_dtype <= SF_BF16,
              SF_EINVAL, "bad rmsnorm dtype");
-  k_rmsnorm<<<rows, kThreads, 0, (hipStream_t)stream>>>(x, delta, w, w_dtype, out, out_dtype, H,
+  const bool wave = delta ? rmsnorm_wave<1>(x, delta, 1, w, w_dtype, out, out_dtype, rows, H, eps, (hipStream_t)stream)
+                          : rmsnorm_wave<0>(x, nullptr, 0, w, w_dtype, out, out_dtype, rows, H, eps,
+                                            (hipStream_t)stream);
+  if (!wave)
+    k_rmsnorm<<<rows, kThreads, 0, (hipStream_t)stream>>>(x, delta, w, w_dtype, out, out_dtype, H,
                                                          eps);
   return sf_check_launch("sf_rmsnorm");
 }
@@ -703,7 +825,8 @@ extern "C" int sf_rmsnorm_partials(float *x, const float *part, int n_parts, con
   SF_REQUIRE(x && part && w && out, SF_EINVAL, "null pointer argument");
   SF_REQUIRE(w_dtype >= SF_F32 && w_dtype <= SF_BF16 && out_dtype >= SF_F32 && out_dtype <= SF_BF16,
              SF_EINVAL, "bad rmsnorm dtype");
-  k_rmsnorm_parts<<<rows, kThreads, 0, (hipStream_t)stream>>>(x, part, n_parts, (size_t)rows * H, w,
+  if (!rmsnorm_wave<2>(x, part, n_parts, w, w_dtype, out, out_dtype, rows, H, eps, (hipStream_t)stream))
+    k_rmsnorm_parts<<<rows, kThreads, 0, (hipStream_t)stream>>>(x, part, n_parts, (size_t)rows * H, w,
                                                               w_dtype, out, out_dtype, H, eps);
   return sf_check_launch("sf_rmsnorm_partials");
 }
@@ -726,10 +849,11 @@ extern "C" int sf_rope_kv_append(const float *qkv, const float *cos_t, const flo
     SF_REQUIRE(pos_host >= 0 && pos_host + rows <= T_cap && pos_host + rows <= max_pos, SF_EINVAL,
                "positions %d..%d exceed the cache capacity %d or the RoPE table %d", pos_host,
                pos_host + rows - 1, T_cap, max_pos);
-  dim3 grid(rows, H + 2 * KVH);
+  const int waves = rope_waves(rows, H + 2 * KVH);
+  dim3 grid(rows, (H + 2 * KVH + waves - 1) / waves);
   const SfRopeAppend a{cos_t, sin_t, max_pos, q_out, q_dtype, k_codes, k_scales, v_codes,
                        v_scales, scale_dtype, H, KVH, D, T_cap};
-  k_rope_kv_append<<<grid, 64, 0, (hipStream_t)stream>>>(qkv, a, pos_dev, pos_host);
+  k_rope_kv_append<<<grid, 64 * waves, 0, (hipStream_t)stream>>>(qkv, a, pos_dev, pos_host);
   return sf_check_launch("sf_rope_kv_append");
 }
 
@@ -756,11 +880,12 @@ extern "C" int sf_rope_kv_append_partials(const float *part, int n_parts, const 
     SF_REQUIRE(pos_host >= 0 && pos_host + rows <= T_cap && pos_host + rows <= max_pos, SF_EINVAL,
                "positions %d..%d exceed the cache capacity %d or the RoPE table %d", pos_host,
                pos_host + rows - 1, T_cap, max_pos);
-  dim3 grid(rows, H + 2 * KVH);
+  const int waves = rope_waves(rows, H + 2 * KVH);
+  dim3 grid(rows, (H + 2 * KVH + waves - 1) / waves);
   const SfRopeAppend a{cos_t, sin_t, max_pos, q_out, q_dtype, k_codes, k_scales, v_codes,
                        v_scales, scale_dtype, H, KVH, D, T_cap};
   const size_t MN = (size_t)rows * (H + 2 * KVH) * D;
-  k_rope_kv_append_parts<<<grid, 64, 0, (hipStream_t)stream>>>(part, n_parts, MN, bias,
+  k_rope_kv_append_parts<<<grid, 64 * waves, 0, (hipStream_t)stream>>>(part, n_parts, MN, bias,
                                                                bias_dtype, a, pos_dev, pos_host);
   return sf_check_launch("sf_rope_kv_append_partials");
 }
