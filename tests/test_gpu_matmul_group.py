@@ -60,7 +60,7 @@ def test_side_by_side(dev, M, Ns, K, g, xdtype, asym):
 @pytest.mark.parametrize("asym", [False, True])
 @pytest.mark.parametrize("xdtype", [torch.float16, torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("M,I,K,g", [(17, 64, 96, 32), (31, 63, 256, 64), (65, 130, 448, 64),
-                                     (200, 1000, 640, 128), (512, 4864, 896, 64)])
+                                     (200, 1000, 640, 128), (512, 4864, 640, 64)])
 def test_swiglu(dev, M, I, K, g, xdtype, asym, packed):
     rng = np.random.default_rng(M + I + K)
     gate, up = _weight(rng, I, K, g, asym), _weight(rng, I, K, g, asym)
@@ -107,3 +107,6 @@ def test_refused_forms(dev):
     assert lib.sf_q4_matmul_group_supported(_lib.SF_GROUP_CONCAT, 2, Ns, 16, 256, 64, _lib.SF_F16, None) == 0
     assert lib.sf_q4_matmul_group_supported(_lib.SF_GROUP_CONCAT, 2, Ns, 64, 256, 48, _lib.SF_F16, None) == 0
     assert lib.sf_q4_matmul_group_supported(_lib.SF_GROUP_CONCAT, 2, Ns, 64, 256, 64, _lib.SF_F16, None) == 1
+    # a weight that splits K by itself keeps its shorter sums
+    Ns = (ctypes.c_int * 2)(4096, 1024)
+    assert lib.sf_q4_matmul_group_supported(_lib.SF_GROUP_CONCAT, 2, Ns, 300, 4096, 64, _lib.SF_F16, None) == 0
