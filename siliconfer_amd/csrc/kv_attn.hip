@@ -453,6 +453,15 @@ __device__ __forceinline__ float sum_x16_x32(float v) {
   p = sf_swap32_pair(v);
   return p.x + p.y;
 }
+// The weights P * V scale as fp16 halves: times 2^10, and less for a query row
+// whose largest weight pm (or V scale vm, in fp32) would overflow.
+constexpr float kVMul = 1024.f, kPvMax = 32768.f;
+// The factor (a power of two) that takes a row's vmul to where they fit.
+__device__ __forceinline__ float fit_shrink(float pm, float vm, float vmul) {
+  float s = 1.f;
+  while ((pm * (vmul * s) > kPvMax || vm * (vmul * s) > 0x1p126f) && vmul * s > 0x1p-20f) s *= 0.25f;
+  return s;
+}
 
 template <int QDT, int SDT, int D, int NW, int NB>
 __global__ void __launch_bounds__(NW * 64)
@@ -1112,10 +1121,15 @@ k_attn_prefill_rows(const void *__restrict__ q, const int8_t *__restrict__ kc,
   };
 
   float m = -INFINITY, lsum = 0.f;  // the row's maximum; this half's share of its sum
-  // The weights P * V scale go to fp16 halves times 2^10 (less where a V scale
-  // would overflow them; powers of two, exact): a weight of 1e-4 at a scale of
-  // 0.02 keeps its low half instead of rounding among fp16's subnormals.
-  float vmul = 1024.f;
+  // The weights P * V scale go to fp16 halves times 2^10 (powers of two, exact):
+  // a weight of 1e-4 at a scale of 0.02 keeps its low half instead of rounding
+  // among fp16's subnormals. A row whose own weights would overflow them takes
+  // less (row_mul): only for keys that it sees, and after the softmax, so that a
+  // large or infinite V scale costs no other row a bit (one factor for the wave
+  // took every row of it down, to zeros). In LDS, where it costs
+  // the rows without one no register.
+  __shared__ float row_mul[NW][32];
+  bool shrunk = false;  // some row's is below 2^10, row_mul holds them all (uniform)
   float16_t O[NDB];
 #pragma unroll
   for (int d = 0; d < NDB; ++d)
@@ -1125,16 +1139,13 @@ k_attn_prefill_rows(const void *__restrict__ q, const int8_t *__restrict__ kc,
   // Loads complete in order: a tile's V is issued before its K and scales, so
   // whoever has the K codes in registers finds V in LDS.
   auto tile = [&](int j, uint8_t *vcur, uint8_t *vnext) {
-    const bool masked = 32 * j + 32 > lo;  // (uniform)
     float sr;
     if constexpr (SDT == SF_F32) sr = sf_bitcast<float>(sbits);
     else sr = (float)sf_bitcast<f16>(sbits);
-    float shrink = 1.f;
-    while (__any(h && fabsf(sr) * vmul > 32768.f && vmul > 0x1p-20f)) {
-      vmul *= 0.25f;
-      shrink *= 0.25f;
-    }
-    scl[wave][h][l32] = sr * (h ? vmul : qscale);
+    // V scales ready to use, or as they are where rows need factors of their own
+    const bool own = shrunk || __any(h && fabsf(sr) * kVMul > kPvMax);
+    const bool masked = own || 32 * j + 32 > lo;  // (uniform)
+    scl[wave][h][l32] = sr * (h ? own ? 1.f : kVMul : qscale);
     load_v(j + NW, vnext);
     __builtin_amdgcn_sched_barrier(0);
     float16_t S = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
@@ -1164,12 +1175,29 @@ k_attn_prefill_rows(const void *__restrict__ q, const int8_t *__restrict__ kc,
     const float2_t mp = sf_swap32_pair(mx);
     const float m_new = fmaxf(m, fmaxf(mp.x, mp.y));
     const float m_ref = m_new == -INFINITY ? 0.f : m_new;
-    if (__any(m_new != m) || shrink != 1.f) {
-      const float cf = __builtin_amdgcn_exp2f(m - m_ref);  // exp2(-inf) = 0
+    float own_mul = 1.f;
+    if (__any(m_new != m) || own) {
+      float cf = __builtin_amdgcn_exp2f(m - m_ref);  // exp2(-inf) = 0
       lsum *= cf;
-#pragma unroll
-      for (int d = 0; d < NDB; ++d) O[d] *= cf * shrink;
       m = m_new;
+      if (own) {
+        const float had = shrunk ? row_mul[wave][l32] : kVMul;
+        float pm = 0.f, vm = 0.f;  // the row's largest weight and V scale
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+          const float v = 8 * (e >> 2) + (e & 3) < left ? fabsf(scl[wave][1][8 * (e >> 2) + 4 * h + (e & 3)]) : 0.f;
+          pm = fmaxf(pm, __builtin_amdgcn_exp2f(sc[e] - m_ref) * v);
+          vm = fmaxf(vm, v);
+        }
+        const float2_t pp = sf_swap32_pair(pm), vp = sf_swap32_pair(vm);
+        const float shrink = fit_shrink(fmaxf(pp.x, pp.y), fmaxf(vp.x, vp.y), had);
+        cf *= shrink;
+        own_mul = had * shrink;
+        row_mul[wave][l32] = own_mul;
+        shrunk = __any(own_mul != kVMul);
+      }
+#pragma unroll
+      for (int d = 0; d < NDB; ++d) O[d] *= cf;
     }
     half8_t ph[2], pl[2];
     float ps = 0.f;
@@ -1178,7 +1206,7 @@ k_attn_prefill_rows(const void *__restrict__ q, const int8_t *__restrict__ kc,
       float4_t v4 = *(const float4_t *)&scl[wave][1][8 * e4 + 4 * h];
       if (masked) {  // masked keys weigh exactly 0 (their scale may be any value)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) v4[i] = 8 * e4 + i < left ? v4[i] : 0.f;
+        for (int i = 0; i < 4; ++i) v4[i] = 8 * e4 + i < left ? v4[i] * own_mul : 0.f;
       }
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
@@ -1224,8 +1252,9 @@ k_attn_prefill_rows(const void *__restrict__ q, const int8_t *__restrict__ kc,
   }
   const float2_t lp = sf_swap32_pair(lsum);
   lsum = lp.x + lp.y;
+  const float unmul = 1.f / (shrunk ? row_mul[wave][l32] : kVMul);
 #pragma unroll
-  for (int d = 0; d < NDB; ++d) O[d] *= 1.f / vmul;
+  for (int d = 0; d < NDB; ++d) O[d] *= unmul;
 
   // ---- merge the wave states pairwise (a wave without tiles holds m = -inf,
   // l = 0, O = 0): waves 2 and 3 into 0 and 1, then 1 into 0, one 32-dim block

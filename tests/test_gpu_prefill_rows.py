@@ -2,8 +2,10 @@
 workgroup per CU) against a float64 evaluation of the same codes and scales:
 row counts around the 32-row blocks and 32-key tiles, with and without a cached
 prefix, both head dims, fp16 / fp32 scales, NaN scales behind the cached length,
-and V scales from tiny to beyond what fp16 weights times 2^10 would hold. q and
-the weights keep 22 bits (two fp16 halves): the bar is 2e-6 of the norm."""
+and V scales from tiny to beyond what fp16 weights times 2^10 would hold, one
+huge or infinite among ordinary ones included: only the rows that see it may
+change. q and the weights keep 22 bits (two fp16 halves): the bar is 2e-6 of the
+norm."""
 
 import numpy as np
 import pytest
@@ -14,7 +16,7 @@ from siliconfer_amd import _lib
 pytestmark = pytest.mark.gpu
 
 
-def run(dev, T, T0, H, KVH, D, qdt, sdt, odt, vscale, dev_pos=False):
+def run(dev, T, T0, H, KVH, D, qdt, sdt, odt, vscale, dev_pos=False, spike=None, faint=False):
     g = torch.Generator(device=dev)
     g.manual_seed(T * 31 + T0 + D)
     n, cap = T0 + T, T0 + T + 3
@@ -24,7 +26,13 @@ def run(dev, T, T0, H, KVH, D, qdt, sdt, odt, vscale, dev_pos=False):
     ks = (0.01 + 0.01 * torch.rand(KVH, cap, generator=g, device=dev)).to(sdt)
     vs = (vscale * (0.5 + torch.rand(KVH, cap, generator=g, device=dev))).to(sdt)
     ks[:, n:], vs[:, n:] = float("nan"), float("nan")  # never-written rows
-    q = (0.7 * r(T, H, D)).to(qdt)
+    q = 0.7 * r(T, H, D)
+    if spike is not None:  # (key, its V scale); faint: a key that every query scores low
+        vs[:, spike[0]] = spike[1]
+        if faint:
+            q += 2
+            kc[:, spike[0]], ks[:, spike[0]] = -127, 0.022
+    q = q.to(qdt)
     out = torch.full((T, H, D), float("nan"), dtype=odt, device=dev)
     st = _lib.stream(q)
     lib = _lib.load()
@@ -77,3 +85,33 @@ def test_rows_v_scale_range(dev, vscale, odt):
     tol = {torch.float32: 4e-6, torch.float16: 2e-2 if vscale < 1e-3 else 1e-3, torch.bfloat16: 4e-3}[odt]
     tol += 8e-9 / vscale
     assert float((out - ref).norm() / ref.norm()) < tol
+
+
+GEO = [(260, 0, 32, 8, 128), (601, 95, 14, 2, 64)]
+
+
+@pytest.mark.parametrize("sdt,value", [(torch.float32, float("inf")), (torch.float16, float("inf")),
+                                       (torch.float32, 1e9), (torch.float32, 1e38)])
+@pytest.mark.parametrize("at", [0, 5, 31, 77, 150, 255])
+@pytest.mark.parametrize("T,T0,H,KVH,D", GEO)
+def test_rows_before_a_large_v_scale(dev, T, T0, H, KVH, D, at, sdt, value):
+    """Rows that do not see the key keep their bits; rows that do meet the bar, or
+    are not finite where the key's weights leave fp16 at every factor (2^10..2^-20)."""
+    args = (dev, T, T0, H, KVH, D, torch.float32, sdt, torch.float32, 0.02)
+    plain, _ = run(*args)
+    out, ref = run(*args, spike=(T0 + at, value))
+    assert torch.equal(out[:at], plain[:at])
+    if value > 1e30:
+        assert not bool(torch.isfinite(out[at:]).any())
+    else:
+        assert float((out[at:] - ref[at:]).norm() / ref[at:].norm()) < 4e-6
+
+
+@pytest.mark.parametrize("T,T0,H,KVH,D", GEO)
+def test_rows_faint_large_v_scale(dev, T, T0, H, KVH, D):
+    """A 1e9 V scale whose key weighs next to nothing takes no bits from the
+    other keys. Its score is -2 * 127 * 0.022 * sqrt(D) = -45 (D = 64) or -63, give
+    or take 127 * 0.022 * 0.7 = 2: its weight times 1e9 stays under 1e-5."""
+    out, ref = run(dev, T, T0, H, KVH, D, torch.float32, torch.float32, torch.float32, 0.02,
+                   spike=(T0 + 40, 1e9), faint=True)
+    assert float((out[41:] - ref[41:]).norm() / ref[41:].norm()) < 2e-6
