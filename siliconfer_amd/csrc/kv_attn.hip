@@ -608,28 +608,37 @@ k_attn_mfma(const void *__restrict__ q, const int8_t *__restrict__ kc, const voi
   for (int d = 0; d < DB; ++d) O[d] = float4_t{0.f, 0.f, 0.f, 0.f};
 
   // Where a wave runs more than one tile, the weights P * V scale go to fp16
-  // halves times 2^10 (less where a V scale would overflow them; powers of two,
-  // exact), so that small weights keep their low half instead of rounding among
-  // fp16's subnormals (error against 64 bits at four sequences of 8191 tokens in
-  // 16 splits: 5.9e-6 without, 3e-7 with). Short runs do without: it costs a
-  // decode step of one tile a wave 0.1 us a launch.
+  // halves times 2^10 (powers of two, exact), so that small weights keep their
+  // low half instead of rounding among fp16's subnormals (error against 64 bits
+  // at four sequences of 8191 tokens in 16 splits: 5.9e-6 without, 3e-7 with).
+  // Less where a V scale would overflow them: fp16 scales at times 1 never do;
+  // an fp32 scale counts by the weights that it makes in the lane's row, not by
+  // its size (a token that weighs next to nothing takes no bits from the
+  // others). Short runs do without: it costs a decode step of one tile a wave
+  // 0.1 us a launch.
   const bool deep = mine > 1;  // (wave-uniform)
-  float vmul = deep ? 1024.f : 1.f;
+  float vmul = deep ? kVMul : 1.f;
 
   auto compute = [&](int j, const Tile &tl) {
     const int tb = 32 * j;
-    float tks[8], tvs[8], vmx = 0.f, shrink = 1.f;
+    float tks[8], tvs[8], shrink = 1.f;
+    bool large = false;  // (wave-uniform)
 #pragma unroll
     for (int r = 0; r < 8; ++r) {
       tks[r] = scale_of(tl.kw, r);
       tvs[r] = scale_of(tl.vw, r);
     }
     if (deep) {
+      float vmx = 0.f;
 #pragma unroll
       for (int r = 0; r < 8; ++r) vmx = fmaxf(vmx, tb + tok_of(r) < Tv ? fabsf(tvs[r]) : 0.f);
-      while (__any(vmx * vmul > 32768.f && vmul > 0x1p-20f)) {
-        vmul *= 0.25f;
-        shrink *= 0.25f;
+      if constexpr (SDT == SF_F32) {
+        large = __any(vmx * vmul > kPvMax);
+      } else {
+        while (__any(vmx * vmul > 65504.f && vmul > 1.f)) {
+          vmul *= 0.25f;
+          shrink *= 0.25f;
+        }
       }
 #pragma unroll
       for (int r = 0; r < 8; ++r) tvs[r] *= vmul;
@@ -660,6 +669,19 @@ k_attn_mfma(const void *__restrict__ q, const int8_t *__restrict__ kc, const voi
     const float m_ref = m_new == -INFINITY ? 0.f : m_new;
     const float c = __builtin_amdgcn_exp2f(m - m_ref);  // exp2(-inf) = 0
     m = m_new;
+    if (SDT == SF_F32 && large) {
+      float pm = 0.f, vm = 0.f;  // the row's largest weight and V scale
+#pragma unroll
+      for (int r = 0; r < 8; ++r) {
+        const float v = tb + tok_of(r) < Tv ? fabsf(scale_of(tl.vw, r)) : 0.f;
+        pm = fmaxf(pm, __builtin_amdgcn_exp2f(sc[r] - m_ref) * v);
+        vm = fmaxf(vm, v);
+      }
+      shrink = fit_shrink(max_x16_x32(pm), max_x16_x32(vm), vmul);
+      vmul *= shrink;
+#pragma unroll
+      for (int r = 0; r < 8; ++r) tvs[r] = scale_of(tl.vw, r) * vmul;
+    }
     half8_t ph, pl;
     float ps = 0.f;
 #pragma unroll
