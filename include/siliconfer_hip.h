@@ -159,8 +159,10 @@ int sf_q4_gemm(const void *blob, const void *x, int x_dtype, void *y, int y_dtyp
                int has_zeros, void *workspace, size_t workspace_bytes, void *stream);
 
 /* Y = X . dequant(W)^T for any M, on whichever kernel is the fastest for the
- * shape: sf_q4_gemv's for few rows (bias may then be y_f32 itself), the tile
- * kernels above that. Arguments and results as sf_q4_gemm. workspace:
+ * shape: sf_q4_gemv's for few rows, the tile kernels above that. Arguments and
+ * results as sf_q4_gemm, but bias may be y_f32 itself, as for sf_q4_gemv (each
+ * output adds its own previous value), for any M: such a call runs as
+ * sf_q4_gemv over 8-row slices. workspace:
  * sf_q4_matmul_workspace_bytes(...) bytes, 16-byte aligned (may be 0 -> NULL
  * ok): K-split partials and, for fp32 X, its bf16 high and low halves. */
 size_t sf_q4_matmul_workspace_bytes(int M, int N, int K, int group_size, int x_dtype);

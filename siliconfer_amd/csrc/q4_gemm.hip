@@ -571,17 +571,22 @@ struct MatmulPlan {
 // 9 to 16 rows stream the weights twice on the GEMV: ahead up to K = 4096 on
 // matrices under 32 M weights (4096 x 4096, 12 rows: 9.7 us against 11.2),
 // behind above (11008 x 4096: 16.7 against 13.9; 1024 x 8192: 14.0 against 11.3).
+// A residual (bias == y_f32: each output adds its own previous value) is the
+// GEMV's form; the tile kernels and the split-K reduce take a bias per column.
 void matmul_plan(int M, int N, int K, int g, bool asym, int xdt, bool residual, MatmulPlan *p) {
   *p = {MatmulPlan::GEMM, 1, 1, 1, 0, 0, 0};
   if (g % 32) return;
+  if (residual) {
+    p->route = MatmulPlan::GEMV;
+    return;
+  }
   sf_gemv::BlkPlan b;
   const bool fits = sf_gemv::plan_blk(M < 8 ? M : 8, N, K, g, xdt, sf_gemv::PRE_NONE, false, &b);
   const bool rows = rows_takes(M, K, g, xdt);
   bool gemv = false;
-  if (M <= 8) gemv = fits && !(rows && !residual && b.kc && xdt == SF_BF16 && g < 128 && (asym || M > 6));
+  if (M <= 8) gemv = fits && !(rows && b.kc && xdt == SF_BF16 && g < 128 && (asym || M > 6));
   else if (M <= kGemmGemvRows)
-    gemv = fits && !residual &&
-           (xdt == SF_F32 || !rows || (K <= 4096 && (size_t)N * K < (size_t)1 << 25));
+    gemv = fits && (xdt == SF_F32 || !rows || (K <= 4096 && (size_t)N * K < (size_t)1 << 25));
   if (gemv) {
     p->route = MatmulPlan::GEMV;
     return;
@@ -639,8 +644,9 @@ static int gemv_slices(const void *blob, const void *x, int x_dtype, void *y, in
     const int mb = M - m0 < 8 ? M - m0 : 8;
     const int rc = sf_q4_gemv(blob, (const char *)x + (size_t)m0 * K * xsz, x_dtype,
                               y ? (char *)y + (size_t)m0 * N * ysz : nullptr, y_dtype,
-                              y_f32 ? y_f32 + (size_t)m0 * N : nullptr, bias, bias_dtype, mb, N, K,
-                              group_size, has_zeros, stream);
+                              y_f32 ? y_f32 + (size_t)m0 * N : nullptr,
+                              bias && bias == (const void *)y_f32 ? y_f32 + (size_t)m0 * N : bias, bias_dtype,
+                              mb, N, K, group_size, has_zeros, stream);
     if (rc) return rc;
   }
   return SF_OK;
@@ -755,14 +761,14 @@ extern "C" int sf_q4_gemm_partials(const void *blob, const void *x, int x_dtype,
                       group_size, has_zeros, workspace, workspace_bytes, stream, true);
 }
 
-// The largest of the plans that has_zeros and a residual bias choose between.
+// The larger of the plans that has_zeros chooses between (a residual needs none).
 extern "C" size_t sf_q4_matmul_workspace_bytes(int M, int N, int K, int group_size, int x_dtype) {
   if (M <= 0 || N <= 0 || K <= 0 || group_size <= 0 || K % group_size) return 0;
   if (x_dtype != SF_F16 && x_dtype != SF_BF16 && x_dtype != SF_F32) return 0;
   size_t bytes = 0;
-  for (int i = 0; i < (M <= kGemmGemvRows ? 4 : 1); ++i) {
+  for (int i = 0; i < (M <= kGemmGemvRows ? 2 : 1); ++i) {
     MatmulPlan p;
-    matmul_plan(M, N, K, group_size, i & 1, x_dtype, i & 2, &p);
+    matmul_plan(M, N, K, group_size, i & 1, x_dtype, false, &p);
     if (p.bytes > bytes) bytes = p.bytes;
   }
   return bytes;

@@ -43,6 +43,26 @@ def test_matmul_tiles(dev, M, N, K, g, xdtype, asym):
     assert np.linalg.norm(y - ref) <= 2e-5 * np.linalg.norm(ref)
 
 
+@pytest.mark.parametrize("M,N,K,g,xdtype", [
+    (3, 4096, 4096, 128, torch.float32), (8, 4096, 4096, 64, torch.float32), (1, 130, 12288, 64, torch.bfloat16),
+    (8, 264, 12288, 64, torch.bfloat16), (9, 1000, 1152, 128, torch.float32), (12, 300, 4224, 64, torch.float16),
+    (17, 129, 320, 32, torch.bfloat16), (40, 257, 1024, 64, torch.float16), (40, 256, 1024, 64, torch.float32),
+    (11, 72, 336, 48, torch.float16)])
+def test_matmul_residual(dev, M, N, K, g, xdtype):
+    """bias == out_f32: every row adds its own previous values, whatever the shape's
+    route without it (rows kernel, K splits, VALU kernel)."""
+    rng = np.random.default_rng(M + N + K)
+    pk, s, z = P.pack_weights_asym(rng.normal(0, 0.02, (N, K)).astype(np.float32), g)
+    w = Q4Weight(pk, s, z, g, device=dev)
+    x = torch.as_tensor(rng.normal(0, 1, (M, K)).astype(np.float32)).to(dev).to(xdtype)
+    h = rng.normal(0, 3, (M, N)).astype(np.float32)
+    y = torch.as_tensor(h).to(dev)
+    w.matmul(x, bias=y, out_f32=y)
+    ref = linear.gemm(pk, s.astype(np.float16).astype(np.float64), x.float().cpu().numpy().astype(np.float64), g,
+                      zeros=z) + h
+    assert np.linalg.norm(y.double().cpu().numpy() - ref) <= 2e-5 * np.linalg.norm(ref)
+
+
 def test_matmul_workspace_is_checked(dev):
     lib = _lib.load()
     M, N, K, g = 40, 256, 1024, 64
