@@ -239,9 +239,15 @@ k_q4_gemm_rows(const std::conditional_t<GRP, RowsGroupArgs, RowsArgs> a) {
   // (64 k) a row; row r's 16-byte piece p sits in place p ^ ((r / 2) % 8), so
   // that 16 rows of one piece (two rows span the 64 banks) touch every bank
   // once; each lane fetches the piece that belongs in its place. Rows past M
-  // repeat row M - 1 (never stored).
-  const __amdgpu_buffer_rsrc_t xrs =
-      __builtin_amdgcn_make_buffer_rsrc((void *)a.x, 0, (SPLIT ? 2 : 1) * M * K * 2, 0x00020000);
+  // repeat row M - 1 (never stored). Rows and lim keep every load inside X. The
+  // resource ends kOver bytes behind it: the range check takes the vector offset
+  // against the size minus the scalar offset (step * 128), which must not wrap
+  // where one row of 2 K bytes is all there is and the last prefetch is up to
+  // 2 (K / 128 + 1) + 3 steps in (holding the scalar offset back instead costs
+  // the loop 1%).
+  constexpr uint32_t kOver = 1024, kPastEnd = 0xC0000000u;
+  const __amdgpu_buffer_rsrc_t xrs = __builtin_amdgcn_make_buffer_rsrc(
+      (void *)a.x, 0, (uint32_t)((SPLIT ? 2 : 1) * M * K * 2) + kOver, 0x00020000);
   uint32_t voff[NF];
   int lim[NF < 2 ? 1 : 2];  // K steps whose piece lies inside K (a last step of 32 k has four)
 #pragma unroll
@@ -260,7 +266,7 @@ k_q4_gemm_rows(const std::conditional_t<GRP, RowsGroupArgs, RowsArgs> a) {
 #pragma unroll
     for (int i = 0; i < NF; ++i)
       load_lds16(xrs, smem + slot * STAGE + (wave * NF + i) * 1024,
-                 step < lim[NF < 2 ? 0 : i & 1] ? voff[i] : 0x80000000u, step * 128);
+                 step < lim[NF < 2 ? 0 : i & 1] ? voff[i] : kPastEnd, step * (R_BK * 2));
   };
 
   // ---- B: the lane's column; a pair of steps is one unit (128 k)

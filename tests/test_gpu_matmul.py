@@ -1,7 +1,7 @@
 """sf_q4_matmul (every kernel it chooses between) against the oracle's GEMM at
-the edges of its tiles: row counts around the GEMV's 8 and 16, the 32-row
-blocks and one to four of them per tile, columns around the 128-wide tiles,
-K of one 32-group, of an odd number of 64-k steps and of several K splits, and
+the edges of its tiles: one row (bf16 with zero-points at long K goes to the rows
+kernel), row counts around the GEMV's 8 and 16, the 32-row blocks and one to
+four of them per tile, columns around the 128-wide tiles, K of one 32-group, of an odd number of 64-k steps and of several K splits, and
 one and two K groups of waves. fp32 sums of exact products: the bar is 2e-5 of
 the result's norm (fp32 activations drop at most 2^-17 of each)."""
 
@@ -16,6 +16,7 @@ from siliconfer_amd.kernels import Q4Weight
 pytestmark = pytest.mark.gpu
 
 SHAPES = [  # M, N, K, g
+    (1, 200, 12288, 64), (1, 4096, 11008, 64), (2, 136, 11008, 64),
     (7, 130, 128, 64), (8, 264, 12288, 64), (9, 1000, 4224, 128), (16, 257, 8192, 64),
     (17, 128, 32, 32), (31, 127, 96, 32), (32, 129, 64, 64), (33, 896, 896, 64),
     (64, 1024, 4096, 128), (65, 300, 320, 64), (95, 2500, 1152, 128), (96, 4864, 896, 64),
