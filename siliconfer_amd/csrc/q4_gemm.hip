@@ -485,9 +485,11 @@ int choose_ksplit(int M, int N, int K) {
 }
 
 // Shapes k_q4_gemm_rows takes: groups of 32, 64 or a multiple of 128, and
-// activations (fp32: both halves) within a buffer resource's 2 GB range.
+// activations (fp32: both halves) within a buffer resource's 2 GB range. fp32
+// rows no more than the grid's 65535 of its 64-row tiles; k_q4_gemm's hold 128,
+// and so do the tiles that 16-bit rows take at such counts.
 bool rows_takes(int M, int K, int g, int xdt) {
-  return (g == 32 || g == 64 || g % 128 == 0) &&
+  return (g == 32 || g == 64 || g % 128 == 0) && (xdt != SF_F32 || M <= 65535 * 64) &&
          (size_t)M * K * (xdt == SF_F32 ? 4 : 2) <= 0x7FFFFFFFu;
 }
 

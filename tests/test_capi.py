@@ -108,6 +108,14 @@ def test_gemm_workspace_and_validation():
 
 
 
+def test_matmul_fp32_rows_within_the_grid():
+    """fp32 rows beyond 65535 tiles of 64 go to the 128-row kernel, which needs no
+    halves of them (M K 4 bytes) in the workspace."""
+    lib = _lib.load()
+    for M, need in ((65535 * 64, 65535 * 64 * 32 * 4), (65535 * 64 + 1, 0), (8_000_000, 0)):
+        assert lib.sf_q4_matmul_workspace_bytes(M, 16, 32, 32, _lib.SF_F32) == need
+
+
 def test_gemm_partials_splits_and_validation():
     """sf_q4_gemm_splits agrees with the workspace sizing (two or more splits
     exactly where sf_q4_gemm needs a workspace of splits x M x N floats);
