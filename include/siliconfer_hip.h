@@ -170,6 +170,10 @@ int sf_q4_matmul(const void *blob, const void *x, int x_dtype, void *y, int y_dt
                  const void *bias, int bias_dtype, int M, int N, int K, int group_size,
                  int has_zeros, void *workspace, size_t workspace_bytes, void *stream);
 
+/* The largest workspace that sf_q4_matmul, sf_q4_gemm or sf_q4_gemm_partials
+ * needs at any M of 1..max_rows (for callers that keep one for every length). */
+size_t sf_q4_rows_workspace_bytes(int max_rows, int N, int K, int group_size, int x_dtype);
+
 /* Several weights of one in_features, group size and zero-point form on the
  * same X in one launch (1 to 3 of them; more than 16 rows):
  *   op SF_GROUP_CONCAT: Y[M][sum N] = their outputs side by side, biases[i]

@@ -52,6 +52,7 @@ _SIGS = {
     "sf_q4_gemm": (_c_i, [_c_p, _c_p, _c_i, _c_p, _c_i, _c_p, _c_p, _c_i,
                           _c_i, _c_i, _c_i, _c_i, _c_i, _c_p, _c_sz, _c_p]),
     "sf_q4_matmul_workspace_bytes": (_c_sz, [_c_i, _c_i, _c_i, _c_i, _c_i]),
+    "sf_q4_rows_workspace_bytes": (_c_sz, [_c_i, _c_i, _c_i, _c_i, _c_i]),
     "sf_q4_matmul": (_c_i, [_c_p, _c_p, _c_i, _c_p, _c_i, _c_p, _c_p, _c_i,
                             _c_i, _c_i, _c_i, _c_i, _c_i, _c_p, _c_sz, _c_p]),
     "sf_q4_matmul_group_supported": (_c_i, [_c_i, _c_i, _c_p, _c_i, _c_i, _c_i, _c_i, _c_p]),

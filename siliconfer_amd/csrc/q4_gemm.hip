@@ -776,6 +776,18 @@ extern "C" size_t sf_q4_matmul_workspace_bytes(int M, int N, int K, int group_si
   return bytes;
 }
 
+extern "C" size_t sf_q4_rows_workspace_bytes(int max_rows, int N, int K, int group_size, int x_dtype) {
+  size_t bytes = 0;
+  for (int m = 0; m < max_rows; ++m) {
+    const int M = m + 1;
+    const size_t a = sf_q4_matmul_workspace_bytes(M, N, K, group_size, x_dtype);
+    const size_t b = sf_q4_gemm_workspace_bytes(M, N, K, group_size);
+    if (a > bytes) bytes = a;
+    if (b > bytes) bytes = b;
+  }
+  return bytes;
+}
+
 extern "C" int sf_q4_matmul(const void *blob, const void *x, int x_dtype, void *y, int y_dtype,
                             float *y_f32, const void *bias, int bias_dtype, int M, int N, int K,
                             int group_size, int has_zeros, void *workspace, size_t workspace_bytes,

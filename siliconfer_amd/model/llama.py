@@ -173,15 +173,12 @@ class LlamaModel:
         self._rows_plans = {}
         self._vbufs = None
         self._prefill_bufs = None
-        # the prefill GEMM's split-K workspace, sized once for every projection
-        # at every chunk length up to max_prefill rows: a recorded verify graph
-        # keeps its address, so it is never replaced
-        ws = 0
-        for w in (L0.qkv, L0.o, L0.gate_up, L0.down):
-            for M in range(1, max(max_prefill, self.VERIFY_ROWS) + 1):
-                ws = max(ws, self._ws_need(w, M),
-                         self.lib.sf_q4_gemm_workspace_bytes(M, w.out_features, w.in_features,
-                                                             w.group_size))
+        # the prompt GEMMs' workspace (K-split partials, fp32 rows' halves), sized
+        # once for every projection at every chunk length up to max_prefill rows:
+        # a recorded verify graph keeps its address, so it is never replaced
+        ws = max(int(self.lib.sf_q4_rows_workspace_bytes(
+            max(max_prefill, self.VERIFY_ROWS), w.out_features, w.in_features, w.group_size, _DT[act_dtype]))
+            for w in (L0.qkv, L0.o, L0.gate_up, L0.down))
         self._gemm_ws = torch.empty(ws, dtype=torch.uint8, device=dev) if ws else None
 
     def sibling(self) -> "LlamaModel":

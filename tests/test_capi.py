@@ -116,6 +116,16 @@ def test_matmul_fp32_rows_within_the_grid():
         assert lib.sf_q4_matmul_workspace_bytes(M, 16, 32, 32, _lib.SF_F32) == need
 
 
+def test_rows_workspace_covers_every_length():
+    lib = _lib.load()
+    for N, K, g in ((896, 4864, 64), (1152, 896, 64), (256, 12288, 64), (100, 336, 48)):
+        for dt in (_lib.SF_F16, _lib.SF_BF16, _lib.SF_F32):
+            each = [max(lib.sf_q4_matmul_workspace_bytes(M, N, K, g, dt), lib.sf_q4_gemm_workspace_bytes(M, N, K, g))
+                    for M in range(1, 130)]
+            for top in (0, 1, 8, 16, 17, 129):
+                assert lib.sf_q4_rows_workspace_bytes(top, N, K, g, dt) == max(each[:top], default=0)
+
+
 def test_gemm_partials_splits_and_validation():
     """sf_q4_gemm_splits agrees with the workspace sizing (two or more splits
     exactly where sf_q4_gemm needs a workspace of splits x M x N floats);
