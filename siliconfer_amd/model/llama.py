@@ -171,6 +171,7 @@ class LlamaModel:
         self.graph = None
         self._verify_graphs = {}
         self._rows_plans = {}
+        self._gemm_plans = {}
         self._vbufs = None
         self._prefill_bufs = None
         # the prompt GEMMs' workspace (K-split partials, fp32 rows' halves), sized
@@ -288,7 +289,7 @@ class LlamaModel:
 
     def _gemm(self, w: Q4Weight, X: torch.Tensor, Y32: torch.Tensor, bias: torch.Tensor | None):
         M = X.shape[0]
-        need = self._ws_need(w, M)
+        need, _ = self._gemm_plan(w, M)
         if need and (self._gemm_ws is None or self._gemm_ws.numel() < need):
             raise SFError(f"GEMM workspace: {need} bytes for {M} rows exceeds the preallocated "
                           f"{0 if self._gemm_ws is None else self._gemm_ws.numel()} (max_prefill)")
@@ -301,24 +302,33 @@ class LlamaModel:
                                         int(w.has_zeros), None if ws is None else ws.data_ptr(),
                                         0 if ws is None else ws.numel(), self._st()), "sf_q4_matmul")
 
-    def _ws_need(self, w: Q4Weight, M: int) -> int:
-        return int(self.lib.sf_q4_matmul_workspace_bytes(M, w.out_features, w.in_features, w.group_size,
-                                                         _DT[self.act_dtype]))
+    def _gemm_plan(self, w: Q4Weight, M: int) -> tuple[int, int]:
+        """(workspace bytes of _gemm, K splits that _gemm_parts leaves or 0) for M
+        rows of a weight of this shape; every layer of a prompt asks."""
+        N, K, g = w.out_features, w.in_features, w.group_size
+        plan = self._gemm_plans.get((M, N, K, g))
+        if plan is None:
+            need = int(self.lib.sf_q4_matmul_workspace_bytes(M, N, K, g, _DT[self.act_dtype]))
+            S = int(self.lib.sf_q4_gemm_splits(M, N, K, g))
+            # Rows that run as batch GEMVs leave no partials. Two splits: the
+            # unsplit tiles of _gemm are faster (512 x 896 x 896 fp16 7.4 us
+            # against 10.1). fp32 activations: _gemm splits them into halves
+            # once, the partials kernel in every tile.
+            if ((M <= GEMM_GEMV_ROWS and self._gemv_ok(min(M, 8), w)) or S <= 2
+                    or self.act_dtype == torch.float32):
+                S = 0
+            plan = self._gemm_plans[(M, N, K, g)] = (need, S)
+        return plan
 
     def _gemm_parts(self, w: Q4Weight, X: torch.Tensor) -> int:
         """Where the GEMM splits K for these rows, run it leaving its partials
         in the GEMM workspace (no reduce launch) and return their count; else
         launch nothing and return 0."""
         M = X.shape[0]
-        if M <= GEMM_GEMV_ROWS and self._gemv_ok(min(M, 8), w):
-            return 0  # sf_q4_gemm runs these rows as 8-row batch GEMVs: no partials
-        S = int(self.lib.sf_q4_gemm_splits(M, w.out_features, w.in_features, w.group_size))
-        # two splits: the unsplit tiles of _gemm are faster (512 x 896 x 896 fp16
-        # 7.4 us against 10.1); fp32 activations: _gemm splits them into halves
-        # once, the partials kernel in every tile
-        if S <= 2 or self.act_dtype == torch.float32:
+        _, S = self._gemm_plan(w, M)
+        if not S:
             return 0
-        need = self.lib.sf_q4_gemm_workspace_bytes(M, w.out_features, w.in_features, w.group_size)
+        need = S * M * w.out_features * 4
         if self._gemm_ws is None or self._gemm_ws.numel() < need:
             raise SFError(f"GEMM workspace: {need} bytes for {M} rows exceeds the preallocated "
                           f"{0 if self._gemm_ws is None else self._gemm_ws.numel()} (max_prefill)")

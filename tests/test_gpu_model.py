@@ -266,3 +266,25 @@ def test_config5_full_workload_against_oracle(dev):
     print(f"config 5: 256 steps checked, {exact} tokens equal to the oracle's argmax, {ties} "
           f"near-ties resolved the other way; worst logit error {worst:.2e} of max |logit|")
     assert exact + ties == 256
+
+
+@pytest.mark.parametrize("T", [5, 13, 40])
+@pytest.mark.parametrize("act", [torch.float32, torch.bfloat16])
+def test_repeated_prompt_asks_for_no_sizes(dev, act, T):
+    """How the projections of T rows run depends on T and the shapes only: the
+    second prompt of a length asks the library for no workspace or split count."""
+    m = LlamaModel.random_init(SMALL, seed=11, group_size=64, device=dev, max_seq=64, act_dtype=act)
+    ids = np.arange(T) % SMALL.vocab_size
+    first = m.prefill(ids)
+    asked, lib = [], m.lib
+
+    class Calls:
+        def __getattr__(self, name):
+            if name.endswith(("_workspace_bytes", "_splits", "_supported")):
+                asked.append(name)
+            return getattr(lib, name)
+
+    m.lib = Calls()
+    m.reset()
+    assert m.prefill(ids) == first
+    assert asked == []
