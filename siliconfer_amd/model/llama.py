@@ -310,12 +310,16 @@ class LlamaModel:
         if plan is None:
             need = int(self.lib.sf_q4_matmul_workspace_bytes(M, N, K, g, _DT[self.act_dtype]))
             S = int(self.lib.sf_q4_gemm_splits(M, N, K, g))
-            # Rows that run as batch GEMVs leave no partials. Two splits: the
-            # unsplit tiles of _gemm are faster (512 x 896 x 896 fp16 7.4 us
-            # against 10.1). fp32 activations: _gemm splits them into halves
-            # once, the partials kernel in every tile.
-            if ((M <= GEMM_GEMV_ROWS and self._gemv_ok(min(M, 8), w)) or S <= 2
-                    or self.act_dtype == torch.float32):
+            # Rows that run as batch GEMVs leave no partials. fp32 activations:
+            # _gemm splits them into halves once, the partials kernel in every
+            # tile. Two splits: partials up to 4 MB, above that _gemm's unsplit
+            # tiles (projection and the RMSNorm or RoPE behind it, fp16, us,
+            # partials / _gemm: 17 x 1152 x 896 7.5 / 10.4, 384 rows 10.9 / 12.0,
+            # 512 rows, 4.7 MB, 13.4 / 12.8; 512 x 896 x 896 9.9 / 10.4; 32 x
+            # 12288 x 4096 17.5 / 18.8, 128 rows 30.7 / 28.3; 384 x 4096 x 2048
+            # 26.0 / 22.3).
+            if ((M <= GEMM_GEMV_ROWS and self._gemv_ok(min(M, 8), w)) or S < 2
+                    or (S == 2 and 8 * M * N > 4 << 20) or self.act_dtype == torch.float32):
                 S = 0
             plan = self._gemm_plans[(M, N, K, g)] = (need, S)
         return plan
@@ -341,7 +345,8 @@ class LlamaModel:
     def _gemm_delta(self, w: Q4Weight, X: torch.Tensor, Dl: torch.Tensor) -> int:
         """The projection's output as the residual's delta: its K-split
         partials left for the next RMSNorm to sum (returns their count), else
-        written to Dl (returns 0). Either way the norm gets the same bits."""
+        written to Dl (returns 0). The two split K differently, so which one runs
+        moves the last bits of the sums."""
         S = self._gemm_parts(w, X)
         if not S:
             self._gemm(w, X, Dl, None)
