@@ -107,8 +107,10 @@ __device__ __forceinline__ uint32_t pk_bf16(float a, float b) {
 // The bf16 B operand of 8 codes (one dword of a unit lane; nibble i is k
 // element 2 i for i < 4, else 2 (i - 4) + 1). Symmetric: (code - 8) / 16, the
 // flipped nibble read as two's complement, 14 VALU instructions (the 16 goes
-// into the group's scale, exactly). With a zero-point: code - z (see
-// q4_gemm.hip), 19.
+// into the group's scale, exactly). With a zero-point, 19: the nibbles go one to
+// a byte, ((b ^ 0x80) - z) ^ 0x80 makes the byte the two's complement of b - z
+// with no borrow between bytes (0x80 + b - z stays in 0x71..0x8F), and each
+// byte converts in one instruction; code - z is exact in bf16.
 template <bool ASYM>
 __device__ __forceinline__ u32x4 dequant_bf16(uint32_t d, uint32_t z) {
   float e0, e1, e2, e3, o0, o1, o2, o3;
@@ -179,15 +181,18 @@ constexpr int rows_lds_bytes() {
 //  * KW = 2: a second set of four waves takes the other half of the K steps and
 //    the sums meet in LDS (two waves a SIMD without a second output tile).
 // The kernel it replaced staged converted codes through LDS with separate
-// convert waves, 128 x 128 tiles only. Measured (us, before -> after): 2048
-// rows on 4096 x 11008, bf16 g128 239 -> 176 (1050 TFLOP/s; torch's bf16 matmul
-// of 8192^3 reaches 1308 on this card), fp16 g128 230 -> 170; 512 on
-// 11008 x 4096, fp16 93 -> 55; 37 on 11008 x 4096, fp16 27 -> 17.5; 512 on
-// 4864 x 896, bf16 with zero-points 13.4 -> 13.4, fp16 16.4 -> 12.7. fp32
-// against the in-kernel split of k_q4_gemm: 333 on 14336 x 4096 191 -> 97.
-// What bounds it at the large end: MFMAs 52% busy, VALU 34%, LDS reads 27% of
-// their cycles without bank conflicts, and a clock of about 1.9-2.0 GHz under
-// this mix (an MFMA-only loop runs at 2.0). Tried and not kept: eight row
+// convert waves, 128 x 128 tiles only. Measured (us a call, before -> after;
+// fp32 results but for the first): 2048 rows on 4096 x 11008, bf16 223 -> 164
+// (1126 TFLOP/s; torch's bf16 matmul of 8192^3 reaches 1308 on this card), fp16
+// 234 -> 173; 512 on 11008 x 4096, fp16 85 -> 58; 48 there 26.1 -> 16.4; 512 on
+// 4864 x 896, bf16 with zero-points 15.9 -> 14.3, fp16 15.3 -> 13.4. fp32 against
+// the in-kernel split of k_q4_gemm: 333 on 11008 x 4096 189 -> 79. Behind that
+// kernel by 1-7%: bf16 with zero-points at K of 8192 and more and 96-333 rows
+// (333 on 4096 x 14336: 74.4 -> 78.0), and 7 units of K on wide weights and
+// 200-333 rows (333 on 9728 x 896 15.5 -> 16.2: two K groups take 8 units' time).
+// What bounds it at the large end (2048 rows on 4096 x 11008, bf16, counters):
+// MFMAs busy 55% of the SIMD cycles and VALU issue 43%, no bank conflicts, at
+// the 1.9 GHz that the card holds under this mix. Tried and not kept: eight row
 // blocks (one wave a SIMD: 234), slot rings of eight with four code sets and a
 // pinned MFMA / VALU interleave (4% slower over the sweep), 256 columns a
 // workgroup (the same).
@@ -240,14 +245,14 @@ k_q4_gemm_rows(const std::conditional_t<GRP, RowsGroupArgs, RowsArgs> a) {
   // that 16 rows of one piece (two rows span the 64 banks) touch every bank
   // once; each lane fetches the piece that belongs in its place. Rows past M
   // repeat row M - 1 (never stored). Rows and lim keep every load inside X. The
-  // resource ends kOver bytes behind it: the range check takes the vector offset
-  // against the size minus the scalar offset (step * 128), which must not wrap
-  // where one row of 2 K bytes is all there is and the last prefetch is up to
-  // 2 (K / 128 + 1) + 3 steps in (holding the scalar offset back instead costs
-  // the loop 1%).
-  constexpr uint32_t kOver = 1024, kPastEnd = 0xC0000000u;
+  // resource ends 1 KB behind it (at most at kPastEnd): the range check takes the
+  // vector offset against the size minus the scalar offset (step * 128), which
+  // must not wrap where one row of 2 K bytes is all there is and the last
+  // prefetch is up to 2 (K / 128 + 1) + 3 steps in (holding the scalar offset
+  // back instead costs the loop 1%).
+  constexpr uint32_t kPastEnd = 0x80000000u;
   const __amdgpu_buffer_rsrc_t xrs = __builtin_amdgcn_make_buffer_rsrc(
-      (void *)a.x, 0, (uint32_t)((SPLIT ? 2 : 1) * M * K * 2) + kOver, 0x00020000);
+      (void *)a.x, 0, min((uint32_t)((SPLIT ? 2 : 1) * M * K * 2) + 1024u, kPastEnd), 0x00020000);
   uint32_t voff[NF];
   int lim[NF < 2 ? 1 : 2];  // K steps whose piece lies inside K (a last step of 32 k has four)
 #pragma unroll
