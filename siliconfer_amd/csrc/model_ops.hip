@@ -113,10 +113,10 @@ k_rmsnorm_parts(float *__restrict__ x, const float *__restrict__ part, int S, si
 // barrier. SfRowNorm's order (its lanes add the same float4s in the same order)
 // and the kernels' arithmetic, so the same bits. SRC: 0 no delta, 1 delta, 2
 // partials. Bound by the latency of one round of loads.
-// Measured (us, looping -> this; no delta / delta / four partials): 1 x 896
-// 3.3 / 3.6 / 3.5 -> 2.4 / 2.5 / 2.9, 512 x 896 3.7 / 4.3 / 4.3 -> 2.8 / 3.2 /
-// 3.6, 1 x 4096 7.4 / 9.8 / 8.3 -> 3.7 / 3.9 / 5.5, 2048 x 4096 16.5 / 28.6 /
-// 43.1 -> 9.8 / 17.6 / 35.6 (5.1, 5.7 and 6.6 TB/s, part of it out of cache).
+// Measured (us, fp16 output, looping -> this; no delta / delta / four partials):
+// 1 x 896 3.1 / 3.5 / 3.5 -> 2.2 / 2.3 / 2.7, 512 x 896 3.6 / 4.2 / 4.3 -> 2.7 /
+// 3.0 / 3.4, 1 x 4096 7.3 / 9.9 / 8.5 -> 3.7 / 3.9 / 5.4, 2048 x 4096 16.1 / 28.6 /
+// 43.7 -> 9.7 / 17.3 / 35.7 (5.2, 6.8 and 6.1 TB/s, part of it out of cache).
 template <int NU, int SRC>
 __global__ void __launch_bounds__(64)
 k_rmsnorm_wave(float *__restrict__ x, const float *__restrict__ delta, int S, size_t MN,

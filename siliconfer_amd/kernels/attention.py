@@ -8,7 +8,7 @@ q [B, H, D]; codes int8 [B, KVH, T, D]; scales [B, KVH, T] or [B, KVH, T, 1]
 (fp32 as the reference stores them, or fp16 as this build's cache does);
 returns float32 [B, H, D]. `n_tiles` is the split-T count with the reference's
 tiling (tile = ceil(T / n_tiles)); by default this build picks its own split
-count for MI355X (`default_splits`, which depends on the head dim) rather than
+count for MI355X (`default_splits`) rather than
 `_choose_n_tiles`, which is kept for callers and tests that use it.
 """
 
@@ -33,8 +33,9 @@ def _choose_n_tiles(T_cache: int, min_tile_size: int = 16, max_tiles: int = 256)
 
 def default_splits(B: int, n_kv_heads: int, T: int, head_dim: int = 64) -> int:
     """The split count `attention_decode` picks when none is given
-    (sf_attn_default_splits_d: one split up to a head_dim-dependent cache
-    length, then about 128 tokens per split)."""
+    (sf_attn_default_splits_d: one split up to 160 cached tokens, then 32 tokens
+    a split up to 2048 and 64 above, 8 to 128 splits; over one workgroup a CU in
+    all sequences and kv heads, one to two a CU)."""
     return int(_lib.load().sf_attn_default_splits_d(B, n_kv_heads, T, head_dim))
 
 

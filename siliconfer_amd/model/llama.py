@@ -35,7 +35,8 @@ from ..kernels.q4 import Q4Weight, matmul_group
 from .config import ModelConfig, rope_tables
 
 _DT = {torch.float32: _lib.SF_F32, torch.float16: _lib.SF_F16, torch.bfloat16: _lib.SF_BF16}
-# sf_q4_gemm runs up to this many rows as 8-row batch GEMVs (no K split)
+# up to this many rows no projection leaves K-split partials (batch GEMVs, or
+# sf_q4_matmul's other kernels), and gate|up and its SwiGLU are launches of their own
 GEMM_GEMV_ROWS = 16
 
 
@@ -294,8 +295,8 @@ class LlamaModel:
             raise SFError(f"GEMM workspace: {need} bytes for {M} rows exceeds the preallocated "
                           f"{0 if self._gemm_ws is None else self._gemm_ws.numel()} (max_prefill)")
         ws = self._gemm_ws if need else None
-        # up to 8 rows (a short chunk, a speculative verify) this is the batch
-        # GEMV, which streams the weights once for all rows
+        # up to 8 rows (a short chunk, a speculative verify) mostly the batch GEMV,
+        # which streams the weights once for all rows
         self._chk(self.lib.sf_q4_matmul(w.blob.data_ptr(), X.data_ptr(), _DT[X.dtype], None, _lib.SF_F32,
                                         Y32.data_ptr(), None if bias is None else bias.data_ptr(),
                                         _lib.SF_F32, M, w.out_features, w.in_features, w.group_size,
@@ -463,7 +464,7 @@ class LlamaModel:
         and return the greedy next token after each of them — the target's
         verify pass of speculative decoding (engine/speculative.py:277-283,
         `t_log = target(verify_ids)`, with the greedy pick of each row). For
-        B <= 8 every projection is one batch GEMV over the B rows, so a
+        B <= 8 every projection is one launch over the B rows, so a
         verify streams the weights once, like one decode step, and after
         `capture_verify()` it is one graph replay. `want_logits` keeps the
         rows' logits in `self.vlogits[:B]` (B <= 8)."""
@@ -550,7 +551,7 @@ class LlamaModel:
 
     def _rows_plan(self, T: int) -> tuple[bool, bool, bool, bool]:
         """How T rows run: (residual, fold_qkv, fold_gate_up, fold_down).
-        residual: up to 8 rows every projection is a batch GEMV and the o /
+        residual: up to 8 rows that the batch GEMV takes in one pass the o /
         down projections add into the residual rows themselves (the norms then
         read them directly). fold_*: the RMSNorm / SwiGLU before that
         projection runs inside it where the GEMV can stage the rows'

@@ -7,8 +7,8 @@ maps [..., in_features] -> [..., out_features] and adds `bias`.
 
 Where the reference evaluates the MLX graph, copies x to the host and runs the
 CPU GEMM on every call (q4_linear.py:51-63), this layer keeps the weights in
-HBM as a repacked blob and runs entirely on the device stream: rows <= 8 go to
-the decode GEMV, more rows to the MFMA prefill GEMM. The output is fp32 like
+HBM as a repacked blob and runs entirely on the device stream: few rows go to
+the decode GEMV, more to the MFMA prefill GEMM (sf_q4_matmul). The output is fp32 like
 the reference's (it casts x to fp32 and its GEMM returns fp32, q4_linear.py:55-63);
 fp16 / bf16 x are read as they are, which equals the reference's upcast since
 every fp16 / bf16 value is exact in fp32. The bias is added in fp32.
